@@ -194,13 +194,13 @@ def profileKernels(enable: bool) -> None:
 
 _KERNEL_SYMBOLS = {
     "gate_up": "moe_gateup_decode_kernel (n <= 4) / dmmv_kernel<T, NT, FUSED=true> / from 16 tokens "
-               "mmq_kernel<T, 1, FUSED=true, SBW> (grouped gate/up + SwiGLU)",
+               "mmw_kernel<T, 1, FUSED=true, ...> (grouped gate/up + SwiGLU)",
     "down": "moe_down_decode_kernel (n <= 4) / dmmv_kernel<T, NT, FUSED=false> / from 16 tokens "
-            "mmq_kernel<T, 1, false, SBW> (grouped down)",
+            "mmw_kernel<T, 1, false, ...> (grouped down)",
     "dense": "dmmv_kernel<T, NT, false> / from 16 vectors mmq_kernel<T, MT, false, SBW> (dense matvec)",
     "attn": "attn_direct_kernel (FAST numerics, more than 4 lanes) / attn_partial_kernel (FAST split-context "
             "attention over the fp16 K/V cache)",
-    "head": "dmmv_kernel<T, NT, false> / from 16 lanes mmq_stream_kernel<T, MT, false> (output head)",
+    "head": "dmmv_kernel<T, NT, false> / from 16 lanes mmw_kernel<T, MT, false, ...> (output head)",
     "qkv": "dmmv_seg_kernel<NT> / from 16 lanes mmq_seg_kernel<1, SBW> (q, k, v in one launch)",
     "wo": "dmmv_kernel<T, NT, false> / from 16 lanes mmq_kernel<T, 1, false, SBW> (wo + residual)",
     "attn_scores": "attn_scores_kernel<HD> (PARITY, up to 4 lanes: dotF32-order scores with the q/k norm, rope and "

@@ -40,7 +40,7 @@ struct DmmvParams {
     int accumulate; // 1: out = out + value (a residual add, tensor.zig:50-52)
     int ident_n;    // launch_mmq only: > 0 means ident_n vectors in groups of consecutive
                     // vectors, identity pair maps, plane 0 -- no group or pair table is read
-    // the streamed gate/up of launch_mmq (mmqs_kernel) only:
+    // launch_mmq's streamed kernel (mmw_kernel) only:
     const int *group_src; // [n_groups][group_stride]: the vector of each group's t-th pair (past n: the
     int group_stride;     // last one's), read in place of pair_src at the group's index; null: pair_src
     int pos_ident;        // pair_dst (and, without group_src, pair_src) is the identity over pair positions

@@ -190,21 +190,19 @@ __device__ __forceinline__ void q6k_tile(const Q6kTile &w, int q4, const mmq_i4 
 // ---- Q4_K with (token, group) rows: up to 16 tokens against unmasked weights -------
 // A 64-deep MFMA span holds two Q4_K groups, each with its own scale.
 // q4k_tile zeroes the weights outside one group and runs one MFMA per group:
-// a masked copy of every weight tile, and a quarter-rate integer multiply
-// per scale.  Here the A rows of an MFMA are (token, group) pairs instead:
-// row m = (t, g) carries token t's activations on the k slots of group part g
-// and zeros elsewhere -- arranged once per token as it loads -- so one MFMA
-// over the unmasked weights returns both groups' integer dots for 8 tokens,
-// and the scales multiply those dots with full-rate 24-bit multiply-adds
-// (|dot| < 2^16, scale <= 63).  The mins are one chained MFMA per span
-// against the part's group min replicated over its k slots: sum_g mn_g *
-// sum(x_g).  Integer dots are exact in any order, so every block's integers
-// -- and the f32 tail after them -- are the reference's.
+// a masked copy of every weight tile, and a multiply per (token, group) of 16
+// tokens however few there are.  Here the A rows of an MFMA are (token, group)
+// pairs instead: row m = (t, g) carries token t's activations on the k slots
+// of group part g and zeros elsewhere, so one MFMA over the unmasked weights
+// returns both groups' integer dots for 8 tokens, and the scales multiply
+// those dots with 24-bit multiply-adds (|dot| < 2^16, scale <= 63).  Integer
+// dots are exact in any order, so every block's integers -- and the f32 tail
+// after them -- are the reference's.
 //
 // k slots.  MFMA (P, half) covers quant spans 2P and 2P + 1: lane
 // quarter q4 holds the 16 bytes 64P + 16*q4 of the block's 128 (span
 // 2P + q4/2, bytes 16*(q4&1) + [0, 16)), their low nibbles for half 0 and
-// high nibbles for half 1 -- group 4P + 2*(q4/2) + half.  A lane loads each
+// high nibbles for half 1 -- group 4P + 2*(q4/2) + half.  A lane reads each
 // weight byte once.  A row r16 = (token r16/2, part r16&1) is nonzero on the
 // quarters with q4/2 == r16&1.
 struct Q4kTileV {
@@ -225,70 +223,6 @@ __device__ __forceinline__ Q4kTileV q4kv_load(const uint8_t *blk, int q4) {
 __device__ __forceinline__ int q4kv_xoff(int j, int q4) {
     return 128 * (j >> 1) + 64 * (q4 >> 1) + 32 * (j & 1) + 16 * (q4 & 1);
 }
-
-// Result lane (row r16, quarter q4) holds A rows 4*q4 + i: tokens 2*q4 + i/2
-// of the set (part i&1), whose two values r[s][0..1] it returns.
-template <int NS>
-__device__ __forceinline__ void q4kv_tile(const Q4kTileV &w, int q4, int ns, const mmq_i4 (&xa)[NS][4],
-                                          const float (&xd)[NS][2], float (&r)[NS][2]) {
-    const uint32_t a = w.hdr.y, b = w.hdr.z, c = w.hdr.w;
-    // Fmt<LH_Q4_K>::scales four groups at a time: bytes 0-3 are groups 0-3 (P = 0), 4-7 (P = 1)
-    const uint32_t scv[2] = {a & 0x3F3F3F3Fu, (c & 0x0F0F0F0Fu) | ((a >> 2) & 0x30303030u)};
-    const uint32_t mnv[2] = {b & 0x3F3F3F3Fu, ((c >> 4) & 0x0F0F0F0Fu) | ((b >> 2) & 0x30303030u)};
-    const float d = half_bits_to_float(w.hdr.x & 0xffff);
-    const float dmin = half_bits_to_float(w.hdr.x >> 16);
-    const mmq_i4 z = {0, 0, 0, 0};
-    // MFMA j = 2P + half: the nibbles (they replace the packed bytes), this
-    // lane's group min replicated (its k slots are group 4P + 2*(q4/2) +
-    // half), and the scales of parts 0 and 1 (groups 4P + half, 4P + 2 + half)
-    mmq_i4 wv[4];
-    int mr[4], s0[4], s1[4];
-#pragma unroll
-    for (int j = 0; j < 4; j++) {
-        const int P = j >> 1, half = j & 1;
-        const uint4 v = w.qs[P];
-        const uint32_t sh = 4 * half;
-        wv[j] = mmq_i4{(int)((v.x >> sh) & 0x0F0F0F0Fu), (int)((v.y >> sh) & 0x0F0F0F0Fu),
-                       (int)((v.z >> sh) & 0x0F0F0F0Fu), (int)((v.w >> sh) & 0x0F0F0F0Fu)};
-        mr[j] = (int)__builtin_amdgcn_perm(mnv[P], mnv[P], (uint32_t)(2 * (q4 >> 1) + half) * 0x01010101u);
-        s0[j] = (int)((scv[P] >> (8 * half)) & 0xFF);
-        s1[j] = (int)((scv[P] >> (8 * (2 + half))) & 0xFF);
-    }
-#pragma unroll
-    for (int s = 0; s < NS; s++) {
-        if (s >= ns)
-            break;
-        mmq_i4 dq[4];
-#pragma unroll
-        for (int j = 0; j < 4; j++)
-            dq[j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(xa[s][j], wv[j], z, 0, 0, 0);
-        mmq_i4 msum = z;
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const mmq_i4 mrep = {mr[j], mr[j], mr[j], mr[j]};
-            msum = __builtin_amdgcn_mfma_i32_16x16x64_i8(xa[s][j], mrep, msum, 0, 0, 0);
-        }
-        int isum[2] = {0, 0};
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            isum[0] += __mul24(s0[j], dq[j][0]) + __mul24(s1[j], dq[j][1]);
-            isum[1] += __mul24(s0[j], dq[j][2]) + __mul24(s1[j], dq[j][3]);
-        }
-#pragma unroll
-        for (int jj = 0; jj < 2; jj++) {
-            // xb.d * (d * f32(isum) - dmin * f32(min_isum))  (ggml.zig:1016-1017)
-            const int ms = msum[2 * jj] + msum[2 * jj + 1];
-            const float aa = d * (float)isum[jj];
-            const float bb = dmin * (float)ms;
-            r[s][jj] = xd[s][jj] * (aa - bb);
-        }
-    }
-}
-
-// LDS row stride of the (token, group) values: a result lane stores tokens
-// 2*q4 + jj of row r16, so the quarters' stores land 2*RS floats apart --
-// 16 or 48 mod 64 (RS = R + 8, R a multiple of 16) puts them in distinct banks.
-__host__ __device__ constexpr int q4kv_rs(int R) { return R + 8; }
 
 // LDS of one work group: the per-block values [FUSED + 1][nb][16*MT][16*RG + 1]
 // (the +1 staggers the four token quarters a wave writes across banks).
@@ -467,401 +401,559 @@ __global__ __launch_bounds__(64 * MMQ_WAVES) void mmq_seg_kernel(DmmvSegParams s
         mmq_body<LH_Q6_K, MT, false, SBW>(p, tile, blockIdx.y, RG, KS, part);
 }
 
-// Streaming variant for one super-block per wave (nb <= MMQ_WAVES): a work
-// group walks NTILE consecutive row tiles of its group (each RG x 16 rows).  The activations are loaded once; each
-// tile's weights are requested while the previous tile computes, in two
-// register sets, and the values meet in two LDS buffers, one barrier per
-// tile.  Same arithmetic and order as mmq_kernel.
-template <int T, int MT, bool FUSED>
-__global__ __launch_bounds__(64 * MMQ_WAVES) void mmq_stream_kernel(DmmvParams p, int RG, int NTILE) {
-    extern __shared__ __align__(16) float part[];
-    constexpr int TOK = 16 * MT;
-    using Tile = typename std::conditional<T == LH_Q4_K, Q4kTile, Q6kTile>::type;
+// ---- streamed in block order --------------------------------------------------------
+// The grouped (expert) matmuls, and lane groups over many rows (the head):
+// bound by the weights' bytes once nothing else is in the way.  A wave owns a
+// 16-row tile for its group's tokens and walks the row's super-blocks in
+// order, so each output is one f32 register that takes `acc += r` block by
+// block: no LDS sums, no barrier between the first block and the last, and
+// the waves of a work group are independent.  Three things decide its speed:
+//   - Loads in address order.  A load whose lanes are in MFMA order (16 rows x
+//     64 bytes, neighbouring lanes in different rows) takes 65 cycles of the
+//     CU's address path per KB, one with neighbouring lanes in one row 18
+//     (probe, L2-resident).  So a wave loads its block with lanes in address
+//     order and turns it into MFMA order through its own LDS.
+//   - Two blocks in registers or in flight while one computes, at 2-4 waves per
+//     SIMD; the tokens' rows staged once per work group with all their loads in
+//     one round trip (staged token by token they took 7 us of a wave's 16).
+//   - Few VALU operations per block: the sets of 8 tokens below, and the mins on
+//     one f16 MFMA.  An int8 MFMA of 16 cycles hides little VALU work (beside
+//     four ANDs of 2.9 cycles it takes 24).
+// Measured (us per launch, rocprof; against the one-shot kernel, the LDS ring
+// that served gate/up over 2048 columns, and the streamed head kernel before):
+// gate/up 7168 -> 2048 over about 60 experts at 24 tokens 434 -> 166, its down
+// 154 -> 84; 2048 -> 768 at 128 tokens 50.6 -> 34.6, down (Q6_K) 51 -> 35; at
+// 32 tokens 26.0 -> 24.9 and 26.9 -> 22.1; the 151936-row Q6_K head at 32
+// lanes 111 -> 81.
+// Q4_K, up to 16 tokens in sets of 8 (token, group part) rows, the arithmetic
+// of q4kv_tile with the mins on one f16 MFMA: sum_g mn_g * sum(x_g) over the
+// block's sixteen 16-value sums, |sum| <= 2032 and mn <= 63 exact in f16, their
+// total below 2^24 exact in f32.  bs: this lane's four sums (A row r16: token
+// mmw_bs_token(r16), sums 4*q4 ..), so result i of a lane is token 8*(i/2) +
+// 2*q4 + (i&1) of its row: the tokens of sets 0 and 1.
+typedef _Float16 mmq_h4 __attribute__((ext_vector_type(4)));
+typedef float mmq_f4 __attribute__((ext_vector_type(4)));
+
+__device__ __forceinline__ int mmw_bs_token(int r16) { return 8 * ((r16 >> 1) & 1) + 2 * (r16 >> 2) + (r16 & 1); }
+
+__device__ __forceinline__ void q4kw_acc(const Q4kTileV &w, int q4, int ns, const mmq_i4 (&xa)[2][4], mmq_h4 bs,
+                                         const float (&xd)[2][2], float (&acc)[2][2]) {
+    const uint32_t a = w.hdr.y, b = w.hdr.z, c = w.hdr.w;
+    const uint32_t scv[2] = {a & 0x3F3F3F3Fu, (c & 0x0F0F0F0Fu) | ((a >> 2) & 0x30303030u)};
+    const uint32_t mnv[2] = {b & 0x3F3F3F3Fu, ((c >> 4) & 0x0F0F0F0Fu) | ((b >> 2) & 0x30303030u)};
+    const float d = half_bits_to_float(w.hdr.x & 0xffff);
+    const float dmin = half_bits_to_float(w.hdr.x >> 16);
+    const mmq_i4 z = {0, 0, 0, 0};
+    const uint32_t m2 = (q4 < 2 ? mnv[0] : mnv[1]) >> (16 * (q4 & 1)); // mins of groups 2*q4, 2*q4 + 1
+    const _Float16 m0 = (_Float16)(unsigned short)(m2 & 0xFF), m1 = (_Float16)(unsigned short)((m2 >> 8) & 0xFF);
+    const mmq_f4 ms = __builtin_amdgcn_mfma_f32_16x16x16f16(bs, mmq_h4{m0, m0, m1, m1}, mmq_f4{0.0f, 0.0f, 0.0f, 0.0f},
+                                                            0, 0, 0);
+    mmq_i4 wv[4];
+    int s0[4], s1[4];
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        const int P = j >> 1, half = j & 1;
+        const uint32_t sh = 4 * half;
+        wv[j] = mmq_i4{(int)((w.qs[P].x >> sh) & 0x0F0F0F0Fu), (int)((w.qs[P].y >> sh) & 0x0F0F0F0Fu),
+                       (int)((w.qs[P].z >> sh) & 0x0F0F0F0Fu), (int)((w.qs[P].w >> sh) & 0x0F0F0F0Fu)};
+        s0[j] = (int)((scv[P] >> (8 * half)) & 0xFF);
+        s1[j] = (int)((scv[P] >> (8 * (2 + half))) & 0xFF);
+    }
+#pragma unroll
+    for (int s = 0; s < 2; s++) {
+        if (s >= ns)
+            break;
+        int isum[2] = {0, 0};
+        mmq_i4 dq[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+            dq[j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(xa[s][j], wv[j], z, 0, 0, 0);
+#pragma unroll
+        for (int j = 0; j < 4; j++) { // 24-bit products (|dot| < 2^16, sc <= 63): exact
+            isum[0] = __mul24(s0[j], dq[j][0]) + isum[0];
+            isum[1] = __mul24(s0[j], dq[j][2]) + isum[1];
+            isum[0] = __mul24(s1[j], dq[j][1]) + isum[0];
+            isum[1] = __mul24(s1[j], dq[j][3]) + isum[1];
+        }
+#pragma unroll
+        for (int jj = 0; jj < 2; jj++) {
+            // xb.d * (d * f32(isum) - dmin * f32(min_isum))  (ggml.zig:1016-1017)
+            const float aa = d * (float)isum[jj];
+            const float bb = dmin * ms[2 * s + jj];
+            acc[s][jj] = acc[s][jj] + xd[s][jj] * (aa - bb);
+        }
+    }
+}
+
+// Q6_K, 16*MT tokens: a lane's 16 values of MFMA h are one run (4h + q4) with
+// one scale, so the scale goes into the weights: v = sc * (q - 32) (14 bits)
+// as the digits v = 128 a + b, a = v >> 7 in [-32, 32] and b = v & 127, each
+// int8.  Two unmasked MFMA chains over the block then give
+// isum = 128 sum(a x) + sum(b x), the reference's integer -- half the MFMAs of
+// one masked MFMA per run, and no multiply per (token, run).
+typedef short mmq_s2 __attribute__((ext_vector_type(2)));
+
+__device__ __forceinline__ void q6k_digits(uint32_t q, mmq_s2 sc, mmq_s2 off, int &hi, int &lo) {
+    // bytes (0, 2) and (1, 3) of q as 16-bit pairs, scaled: sc * q - 32 sc
+    const mmq_s2 e = __builtin_bit_cast(mmq_s2, q & 0x00FF00FFu) * sc + off;
+    const mmq_s2 o = __builtin_bit_cast(mmq_s2, (q >> 8) & 0x00FF00FFu) * sc + off;
+    const mmq_s2 eh = e >> 7, oh = o >> 7;
+    // result byte k = low byte of value k: e.lo, o.lo, e.hi, o.hi
+    hi = (int)__builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, oh), __builtin_bit_cast(uint32_t, eh), 0x06020400u);
+    lo = (int)(__builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, o), __builtin_bit_cast(uint32_t, e), 0x06020400u) &
+               0x7F7F7F7Fu);
+}
+
+template <int MT>
+__device__ __forceinline__ void q6kw_acc(const Q6kTile &w, int q4, const mmq_i4 (&xa)[MT][4],
+                                         const float4 (&xd)[MT], float (&acc)[MT][4]) {
+    const float dw = half_bits_to_float(w.d);
+    const mmq_i4 z = {0, 0, 0, 0};
+    const uint32_t scw[4] = {w.sc.x, w.sc.y, w.sc.z, w.sc.w};
+    mmq_i4 ah[MT], al[MT];
+#pragma unroll
+    for (int mt = 0; mt < MT; mt++)
+        ah[mt] = al[mt] = z;
+#pragma unroll
+    for (int h = 0; h < 4; h++) {
+        const int n = h >> 1, ls = 4 * (h & 1), hs = 4 * (h & 1) + 2 * (q4 >> 1);
+        const short sc = (short)(int8_t)((scw[h] >> (8 * q4)) & 0xFF);
+        const mmq_s2 s2 = {sc, sc};
+        mmq_s2 off = s2 * (short)-32;
+        asm("" : "+v"(off)); // kept a value of its own: one packed multiply-add per pair below
+        const uint32_t ql[4] = {w.ql[n].x, w.ql[n].y, w.ql[n].z, w.ql[n].w};
+        const uint32_t qh[4] = {w.qh[n].x, w.qh[n].y, w.qh[n].z, w.qh[n].w};
+        mmq_i4 whi, wlo;
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            int hi, lo;
+            q6k_digits(((ql[e] >> ls) & 0x0F0F0F0Fu) | (((qh[e] >> hs) & 0x03030303u) << 4), s2, off, hi, lo);
+            whi[e] = hi;
+            wlo[e] = lo;
+        }
+#pragma unroll
+        for (int mt = 0; mt < MT; mt++) {
+            ah[mt] = __builtin_amdgcn_mfma_i32_16x16x64_i8(xa[mt][h], whi, ah[mt], 0, 0, 0);
+            al[mt] = __builtin_amdgcn_mfma_i32_16x16x64_i8(xa[mt][h], wlo, al[mt], 0, 0, 0);
+        }
+    }
+#pragma unroll
+    for (int mt = 0; mt < MT; mt++) {
+        const float xs[4] = {xd[mt].x, xd[mt].y, xd[mt].z, xd[mt].w};
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            // xb.d * dec.d * f32(isum)  (ggml.zig:1019)
+            const float s = xs[i] * dw;
+            acc[mt][i] = acc[mt][i] + s * (float)((ah[mt][i] << 7) + al[mt][i]);
+        }
+    }
+}
+
+// One block of 16 rows, as loaded (lanes in address order) and as kept in LDS.
+// LDS holds a row's 16-byte chunks one after another (Q4_K: the 9 of its
+// GGML block; Q6_K: 8 of ql, 4 of qh, the scales; d apart): odd chunk
+// strides, so the 16 rows a wave reads together sit in different banks.
+// Src: the lane's byte offsets in the tile's rows (rows past the last read that
+// one).
+template <int T> struct MmwBlk;
+template <> struct MmwBlk<LH_Q4_K> {
+    static constexpr int ROWB = 144, BYTES = 16 * 144;
+    using Tile = Q4kTileV;
+    mmq_i4 v0, v1;
+    uint32_t t; // chunks 128 .. 143 of the 144, a dword per lane
+    struct Src {
+        const uint8_t *b;
+        uint32_t o[3];
+    };
+    __device__ __forceinline__ static Src src(const uint8_t *wb, size_t, int rows, int nb, int row0, int ln) {
+        Src s;
+        s.b = wb;
+#pragma unroll
+        for (int i = 0; i < 3; i++) {
+            const int q = i < 2 ? 64 * i + ln : 128 + (ln >> 2);
+            const int r = q / 9, c = q - 9 * r;
+            s.o[i] = (uint32_t)min(row0 + r, rows - 1) * (uint32_t)(nb * 144) + 16 * c + (i == 2 ? 4 * (ln & 3) : 0);
+        }
+        return s;
+    }
+    __device__ __forceinline__ void load(const Src &s, int b) {
+        const uint8_t *p = s.b + (size_t)b * 144;
+        v0 = *(const mmq_i4 *)(p + s.o[0]);
+        v1 = *(const mmq_i4 *)(p + s.o[1]);
+        t = *(const uint32_t *)(p + s.o[2]);
+    }
+    __device__ __forceinline__ void store(uint8_t *l, int ln) const {
+        *(mmq_i4 *)(l + 16 * ln) = v0;
+        *(mmq_i4 *)(l + 1024 + 16 * ln) = v1;
+        *(uint32_t *)(l + 2048 + 4 * ln) = t;
+    }
+    __device__ __forceinline__ static Tile tile(const uint8_t *l, int r16, int q4) {
+        return q4kv_load(l + r16 * ROWB, q4);
+    }
+};
+template <> struct MmwBlk<LH_Q6_K> {
+    static constexpr int ROWB = 208, BYTES = 16 * 208 + 64;
+    using Tile = Q6kTile;
+    mmq_i4 v0, v1, v2; // ql chunks 0-63, 64-127 of the 16 rows, qh
+    uint32_t s, d;
+    struct Src {
+        const uint8_t *q, *h, *sc, *d;
+        uint32_t oq0, oq1, oh, os, od;
+    };
+    __device__ __forceinline__ static Src src(const uint8_t *wb, size_t U, int rows, int nb, int row0, int ln) {
+        Src s;
+        s.q = wb;
+        s.h = wb + U * 128;
+        s.sc = wb + U * 192;
+        s.d = wb + U * 208;
+        const uint32_t u0 = (uint32_t)min(row0 + (ln >> 3), rows - 1) * nb;
+        const uint32_t u1 = (uint32_t)min(row0 + 8 + (ln >> 3), rows - 1) * nb;
+        const uint32_t u2 = (uint32_t)min(row0 + (ln >> 2), rows - 1) * nb;
+        s.oq0 = u0 * 128 + 16 * (ln & 7);
+        s.oq1 = u1 * 128 + 16 * (ln & 7);
+        s.oh = u2 * 64 + 16 * (ln & 3);
+        s.os = u2 * 16 + 4 * (ln & 3);
+        s.od = u2 * 2;
+        return s;
+    }
+    __device__ __forceinline__ void load(const Src &s_, int b) {
+        v0 = *(const mmq_i4 *)(s_.q + (size_t)b * 128 + s_.oq0);
+        v1 = *(const mmq_i4 *)(s_.q + (size_t)b * 128 + s_.oq1);
+        v2 = *(const mmq_i4 *)(s_.h + (size_t)b * 64 + s_.oh);
+        s = *(const uint32_t *)(s_.sc + (size_t)b * 16 + s_.os);
+        d = *(const uint16_t *)(s_.d + (size_t)b * 2 + s_.od);
+    }
+    __device__ __forceinline__ void store(uint8_t *l, int ln) const {
+        *(mmq_i4 *)(l + (ln >> 3) * ROWB + 16 * (ln & 7)) = v0;
+        *(mmq_i4 *)(l + (8 + (ln >> 3)) * ROWB + 16 * (ln & 7)) = v1;
+        *(mmq_i4 *)(l + (ln >> 2) * ROWB + 128 + 16 * (ln & 3)) = v2;
+        *(uint32_t *)(l + (ln >> 2) * ROWB + 192 + 4 * (ln & 3)) = s;
+        *(uint32_t *)(l + 16 * ROWB + 4 * (ln >> 2)) = d;
+    }
+    __device__ __forceinline__ static Tile tile(const uint8_t *l, int r16, int q4) {
+        Tile w;
+        const uint8_t *p = l + r16 * ROWB;
+#pragma unroll
+        for (int n = 0; n < 2; n++) {
+            w.ql[n] = *(const uint4 *)(p + 64 * n + 16 * q4);
+            w.qh[n] = *(const uint4 *)(p + 128 + 32 * n + 16 * (q4 & 1));
+        }
+        w.sc = *(const uint4 *)(p + 192);
+        w.d = (uint16_t) * (const uint32_t *)(l + 16 * ROWB + 4 * r16);
+        return w;
+    }
+};
+
+// Orders this wave's LDS stores against its own reads by other lanes (the
+// LDS serves a wave's accesses in order; this keeps the compiler's order).
+__device__ __forceinline__ void wave_lds_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+}
+
+constexpr int MMW_W = 4;          // waves per work group: four neighbouring row tiles, four staged tokens each
+constexpr int MMW_XL_COLS = 2048; // the tokens' whole rows are staged in LDS up to here
+
+// LDS of a work group: scales [nb][TOK]; the tokens' rows [TOK][xrow] (Q4_K:
+// then 256 zeros and the 16-value sums [TOK][brow]) once (XL) or one block
+// of them per wave; per wave a block of 16 weight rows.
+template <int T, int MT, bool XL>
+__host__ __device__ constexpr int mmw_xbytes(int cols) {
+    const int xrow = (XL ? cols : 256) + 16, brow = (XL ? cols / 256 : 1) * 32 + 16;
+    return 16 * MT * xrow + (T == LH_Q4_K ? 256 + 16 * MT * brow : 0);
+}
+template <int T, int MT, bool XL>
+static size_t mmw_lds(int cols) {
+    const size_t x = mmw_xbytes<T, MT, XL>(cols);
+    return (size_t)(cols / 256) * 64 * MT + (XL ? x + MMW_W * MmwBlk<T>::BYTES : MMW_W * (x + MmwBlk<T>::BYTES));
+}
+
+// FUSED: gate and up with the SwiGLU epilogue.  XL: the tokens' int8 rows are
+// staged in LDS once per work group; else each wave brings a block's columns of
+// them along with the block's weights.
+template <int T, int MT, bool FUSED, bool XL, int OCC>
+__global__ __launch_bounds__(64 * MMW_W, OCC) void mmw_kernel(DmmvParams p) {
+    extern __shared__ __align__(16) uint8_t sh[];
+    using B = MmwBlk<T>;
+    constexpr bool K4 = T == LH_Q4_K;
+    static_assert(!K4 || MT == 1, "Q4_K: 16 tokens");
+    static_assert(!FUSED || K4, "a fused pair is Q4_K");
+    constexpr int TOK = 16 * MT, M = FUSED ? 2 : 1, W = MMW_W, XN = 4 * MT;
     const bool ident = p.ident_n > 0;
+    const int cols = p.cols, nb = cols / 256;
+    const int gi = blockIdx.y;
     DmmvGroup grp;
     if (ident) {
         grp.plane = 0;
-        grp.first = (int)blockIdx.y * TOK;
+        grp.first = gi * TOK;
         grp.n = min(TOK, p.ident_n - grp.first);
     } else {
         const int ng = p.n_groups_dev ? *p.n_groups_dev : p.n_groups;
-        if ((int)blockIdx.y >= ng)
+        if (gi >= ng)
             return;
-        grp = p.groups[blockIdx.y];
+        grp = p.groups[gi];
     }
-    const int n = grp.n, cols = p.cols, nb = cols / 256;
+    const int n = grp.n, ns = (n + 7) / 8; // Q4_K: sets of 8 tokens
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), ln = threadIdx.x & 63;
     const int r16 = ln & 15, q4 = ln >> 4;
-    const int rg = wave % RG, b = wave / RG; // this wave's super-block
-    const int R = 16 * RG, RS = R + 1;
-    const int rl = 16 * rg + r16;
-    const int tile0 = blockIdx.x * NTILE;
-    const int nti = min(NTILE, (p.rows + R - 1) / R - tile0);
-    const size_t U = (size_t)p.rows * nb;
-    const size_t mat = (size_t)nb * TOK * RS;
-    const size_t buf = (size_t)(FUSED ? 2 : 1) * mat;
-    const uint8_t *wb = p.w + (size_t)grp.plane * p.plane_bytes;
-    const uint8_t *wb2 = FUSED ? p.w2 + (size_t)grp.plane * p.plane_bytes : nullptr;
-    auto load_tile = [&](int tile, Tile &a, Tile &a2) {
-        const size_t unit = (size_t)min(tile * R + rl, p.rows - 1) * nb + b;
-        if constexpr (T == LH_Q4_K) {
-            a = q4k_load(wb + unit * 144, q4);
-            if constexpr (FUSED)
-                a2 = q4k_load(wb2 + unit * 144, q4);
-        } else {
-            a = q6k_load(wb, U, unit, q4);
+    const int row0 = ((int)blockIdx.x * W + wave) * 16;
+    const int xrow = (XL ? cols : 256) + 16, brow = (XL ? nb : 1) * 32 + 16;
+    const int xbytes = mmw_xbytes<T, MT, XL>(cols);
+    float *xds = (float *)sh;
+    uint8_t *wls = sh + (size_t)nb * TOK * 4 + (XL ? xbytes + wave * B::BYTES : wave * (B::BYTES + xbytes));
+    uint8_t *xl = XL ? sh + (size_t)nb * TOK * 4 : wls + B::BYTES;
+    uint8_t *zl = xl + TOK * xrow, *bl = zl + 256;
+    auto halves = [](const mmq_i4 &v) {
+        return mmq_h4{(_Float16)(short)v[0], (_Float16)(short)v[1], (_Float16)(short)v[2], (_Float16)(short)v[3]};
+    };
+    // the vector of the group's t-th token (past n: the last); group_src needs no group
+    const int *tab = p.group_src ? p.group_src + (size_t)gi * p.group_stride : p.pair_src + grp.first;
+    const int tmax = p.group_src ? TOK - 1 : n - 1;
+    auto vec_of = [&](int t) { return tab[min(t, tmax)]; };
+    typename B::Src src[M];
+    src[0] = B::src(p.w + (size_t)grp.plane * p.plane_bytes, (size_t)p.rows * nb, p.rows, nb, row0, ln);
+    if constexpr (FUSED) {
+        src[1] = src[0];
+        src[1].b = p.w2 + (size_t)grp.plane * p.plane_bytes;
+    }
+    struct Stage {
+        B w[M];
+        mmq_i4 x[XL ? 1 : XN], bs; // (not XL) tokens 4 i + ln / 16, chunk ln % 16; sums 4 (ln % 4) .. of token ln / 4
+    } st[2];
+    const int8_t *xr[XN];
+    const int32_t *br;
+    if constexpr (!XL) {
+#pragma unroll
+        for (int i = 0; i < XN; i++)
+            xr[i] = p.xq + (size_t)vec_of(4 * i + (ln >> 4)) * cols + 16 * (ln & 15);
+        if constexpr (K4)
+            br = p.xs + (size_t)vec_of(ln >> 2) * (cols / 16) + 4 * (ln & 3);
+    }
+    auto load = [&](Stage &s, int b) {
+        s.w[0].load(src[0], b);
+        if constexpr (FUSED)
+            s.w[1].load(src[1], b);
+        if constexpr (!XL) {
+#pragma unroll
+            for (int i = 0; i < XN; i++)
+                s.x[i] = *(const mmq_i4 *)(xr[i] + 256 * b);
+            if constexpr (K4)
+                s.bs = *(const mmq_i4 *)(br + 16 * b);
         }
     };
-    Tile wa, wa2, wbt, wbt2;
-    load_tile(tile0, wa, wa2);
-    int vrow[MT];
+    auto commit = [&](const Stage &s, int m) { // matrix m's block to this wave's LDS
+        wave_lds_sync();
+        s.w[m].store(wls, ln);
+        if constexpr (!XL)
+            if (m == 0) {
+#pragma unroll
+                for (int i = 0; i < XN; i++)
+                    *(mmq_i4 *)(xl + (4 * i + (ln >> 4)) * xrow + 16 * (ln & 15)) = s.x[i];
+                if constexpr (K4)
+                    *(mmq_h4 *)(bl + (ln >> 2) * brow + 8 * (ln & 3)) = halves(s.bs);
+            }
+        wave_lds_sync();
+    };
+    // the block scales: 16 threads per token
+    const int xt16 = threadIdx.x >> 4, xb16 = threadIdx.x & 15;
+    const float *xdp[MT];
 #pragma unroll
     for (int mt = 0; mt < MT; mt++)
-        vrow[mt] = ident ? grp.first + min(16 * mt + r16, n - 1) : p.pair_src[grp.first + min(16 * mt + r16, n - 1)];
-    mmq_i4 xa[MT][4];
-    float xd[MT][4];
+        xdp[mt] = p.xd + (size_t)vec_of(16 * mt + xt16) * nb;
+    if constexpr (XL) {
+        // nb <= 8: XN token rows per wave, all their loads before the weights' and
+        // the stores behind them, so one round trip covers the staging
+        int v[XN];
 #pragma unroll
-    for (int mt = 0; mt < MT; mt++) {
-        const int8_t *xr = p.xq + (size_t)vrow[mt] * cols + 256 * b + 16 * q4;
+        for (int i = 0; i < XN; i++)
+            v[i] = vec_of(XN * wave + i);
+        const int c0 = min(ln, 16 * nb - 1), c1 = min(64 + ln, 16 * nb - 1);
+        mmq_i4 x0[XN], x1[XN], bs[2];
+        float xdv[MT];
 #pragma unroll
-        for (int s4 = 0; s4 < 4; s4++)
-            xa[mt][s4] = *(const mmq_i4 *)(xr + 64 * s4);
-#pragma unroll
-        for (int i = 0; i < 4; i++)
-            xd[mt][i] = p.xd[(size_t)__shfl(vrow[mt], 4 * q4 + i) * nb + b];
-    }
-    // one tile: its values into LDS buffer pb, the barrier, then the outputs
-    auto run_tile = [&](int it, const Tile &w, const Tile &w2) {
-        float *pb = part + (size_t)(it & 1) * buf;
-        float r[MT][4], r2[MT][4];
-        if constexpr (T == LH_Q4_K) {
-            q4k_tile<MT>(w, q4, xa, xd, r);
-            if constexpr (FUSED)
-                q4k_tile<MT>(w2, q4, xa, xd, r2);
-        } else {
-            q6k_tile<MT>(w, q4, xa, xd, r);
+        for (int i = 0; i < XN; i++) {
+            x0[i] = *(const mmq_i4 *)(p.xq + (size_t)v[i] * cols + 16 * c0);
+            x1[i] = *(const mmq_i4 *)(p.xq + (size_t)v[i] * cols + 16 * c1);
+        }
+        if constexpr (K4) {
+            const int va = ln < 32 ? v[0] : v[1], vb = ln < 32 ? v[2] : v[3], cb = min(ln & 31, 4 * nb - 1);
+            bs[0] = *(const mmq_i4 *)(p.xs + (size_t)va * (cols / 16) + 4 * cb);
+            bs[1] = *(const mmq_i4 *)(p.xs + (size_t)vb * (cols / 16) + 4 * cb);
         }
 #pragma unroll
         for (int mt = 0; mt < MT; mt++)
+            xdv[mt] = xdp[mt][min(xb16, nb - 1)];
+        __builtin_amdgcn_sched_barrier(0);
+        load(st[0], 0);
+        load(st[1], min(1, nb - 1));
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const size_t o = ((size_t)b * TOK + 16 * mt + 4 * q4 + i) * RS + rl;
-                pb[o] = r[mt][i];
-                if constexpr (FUSED)
-                    pb[mat + o] = r2[mt][i];
+        for (int i = 0; i < XN; i++) {
+            uint8_t *l = xl + (size_t)(XN * wave + i) * xrow;
+            if (ln < 16 * nb)
+                *(mmq_i4 *)(l + 16 * ln) = x0[i];
+            if (64 + ln < 16 * nb)
+                *(mmq_i4 *)(l + 16 * (64 + ln)) = x1[i];
+        }
+        if constexpr (K4)
+#pragma unroll
+            for (int i = 0; i < 2; i++)
+                if ((ln & 31) < 4 * nb)
+                    *(mmq_h4 *)(bl + (size_t)(4 * wave + 2 * i + (ln >> 5)) * brow + 8 * (ln & 31)) = halves(bs[i]);
+#pragma unroll
+        for (int mt = 0; mt < MT; mt++)
+            if (xb16 < nb)
+                xds[xb16 * TOK + 16 * mt + xt16] = xdv[mt];
+        if (K4 && threadIdx.x < 16)
+            *(mmq_i4 *)(zl + 16 * threadIdx.x) = mmq_i4{0, 0, 0, 0};
+    } else {
+        load(st[0], 0);
+        load(st[1], min(1, nb - 1));
+        for (int b0 = 0; b0 < nb; b0 += 64) {
+            float v[MT][4];
+#pragma unroll
+            for (int mt = 0; mt < MT; mt++)
+#pragma unroll
+                for (int u = 0; u < 4; u++)
+                    v[mt][u] = xdp[mt][min(b0 + 16 * u + xb16, nb - 1)];
+#pragma unroll
+            for (int mt = 0; mt < MT; mt++)
+#pragma unroll
+                for (int u = 0; u < 4; u++)
+                    if (b0 + 16 * u + xb16 < nb)
+                        xds[(b0 + 16 * u + xb16) * TOK + 16 * mt + xt16] = v[mt][u];
+        }
+        if (K4 && ln < 16)
+            *(mmq_i4 *)(zl + 16 * ln) = mmq_i4{0, 0, 0, 0};
+    }
+    lds_barrier();
+    // Q4_K: A row r16 = (token r16/2 of the set, group part r16&1): live on the
+    // quarters of its part, zeros elsewhere; Q6_K: token r16
+    const bool live = (q4 >> 1) == (r16 & 1);
+    const int xstep = XL && (live || !K4) ? 256 : 0;
+    const uint8_t *xt[2], *bt = bl + mmw_bs_token(r16) * brow + 8 * q4;
+    if constexpr (K4) {
+        xt[0] = live ? xl + (r16 / 2) * xrow : zl;
+        xt[1] = live ? xl + (8 + r16 / 2) * xrow : zl;
+    } else {
+        xt[0] = xl + r16 * xrow + 16 * q4;
+        xt[1] = xl + (MT == 2 ? 16 + r16 : r16) * xrow + 16 * q4;
+    }
+    // accumulators: Q4_K [matrix][set][token pair], Q6_K [0][token tile][4 tokens]
+    float acc4[M][2][2] = {}, acc6[MT][4] = {};
+    // Block b: its A rows from LDS, then each matrix's MFMAs with the next
+    // tile (the other matrix, or the next block) already stored to LDS and
+    // read back in MFMA order, so that latency runs under the arithmetic.
+    commit(st[0], 0);
+    typename B::Tile w0 = B::tile(wls, r16, q4);
+    auto step = [&](int b, Stage &cur, const Stage &nxt) {
+        if constexpr (K4) {
+            mmq_i4 xa[2][4];
+            float xd[2][2];
+#pragma unroll
+            for (int s = 0; s < 2; s++) {
+                if (s >= ns)
+                    break;
+#pragma unroll
+                for (int j = 0; j < 4; j++)
+                    xa[s][j] = *(const mmq_i4 *)(xt[s] + b * xstep + q4kv_xoff(j, q4));
+                const float2 v = *(const float2 *)(xds + b * TOK + 8 * s + 2 * q4);
+                xd[s][0] = v.x;
+                xd[s][1] = v.y;
             }
-        // a buffer is written again two tiles on, after every thread has
-        // passed the next tile's barrier
-        __syncthreads();
-        const int row0 = (tile0 + it) * R;
-        for (int idx = threadIdx.x; idx < n * R; idx += blockDim.x) {
-            const int tk = idx / R, rr = idx % R;
-            if (row0 + rr >= p.rows)
-                continue;
-            const float *pv = pb + (size_t)tk * RS + rr;
-            float acc = 0.0f;
-            for (int bb = 0; bb < nb; bb++)
-                acc = acc + pv[(size_t)bb * TOK * RS];
-            float v = acc;
+            const mmq_h4 bs = *(const mmq_h4 *)(bt + (XL ? 32 * b : 0));
+            commit(FUSED ? cur : nxt, FUSED ? 1 : 0);
+            const Q4kTileV w1 = B::tile(wls, r16, q4);
+            load(cur, min(b + 2, nb - 1)); // past the last block: the last one again, not used
+            __builtin_amdgcn_sched_barrier(0);
+            q4kw_acc(w0, q4, ns, xa, bs, xd, acc4[0]);
             if constexpr (FUSED) {
-                float acc2 = 0.0f;
-                for (int bb = 0; bb < nb; bb++)
-                    acc2 = acc2 + pv[mat + (size_t)bb * TOK * RS];
-                v = swiglu1(acc, acc2);
+                commit(nxt, 0);
+                w0 = B::tile(wls, r16, q4);
+                q4kw_acc(w1, q4, ns, xa, bs, xd, acc4[M - 1]);
+            } else {
+                w0 = w1;
             }
-            const int dst = ident ? grp.first + tk : p.pair_dst[grp.first + tk];
-            float *o = p.out + (size_t)dst * p.out_stride + row0 + rr;
-            *o = p.accumulate ? *o + v : v;
+        } else {
+            float4 xd[MT];
+            mmq_i4 xa[MT][4];
+#pragma unroll
+            for (int mt = 0; mt < MT; mt++) {
+                xd[mt] = *(const float4 *)(xds + b * TOK + 16 * mt + 4 * q4);
+#pragma unroll
+                for (int j = 0; j < 4; j++)
+                    xa[mt][j] = *(const mmq_i4 *)(xt[mt] + b * xstep + 64 * j);
+            }
+            commit(nxt, 0);
+            const typename B::Tile w1 = B::tile(wls, r16, q4);
+            load(cur, min(b + 2, nb - 1)); // past the last block: the last one again, not used
+            __builtin_amdgcn_sched_barrier(0);
+            q6kw_acc<MT>(w0, q4, xa, xd, acc6);
+            w0 = w1;
         }
     };
-    for (int it = 0; it < nti; it += 2) {
-        if (it + 1 < nti)
-            load_tile(tile0 + it + 1, wbt, wbt2);
-        __builtin_amdgcn_sched_barrier(0);
-        run_tile(it, wa, wa2);
-        if (it + 1 >= nti)
+    for (int b = 0; b < nb; b += 2) {
+        step(b, st[0], st[1]);
+        if (b + 1 >= nb)
             break;
-        if (it + 2 < nti)
-            load_tile(tile0 + it + 2, wa, wa2);
-        __builtin_amdgcn_sched_barrier(0);
-        run_tile(it + 1, wbt, wbt2);
+        step(b + 1, st[1], st[0]);
     }
-}
-
-// ---- grouped Q4_K expert matmuls streamed through LDS ------------------------------
-// The one-shot work groups of mmq_kernel hold their weights in registers from
-// the first load to the last MFMA: two of them fit a CU, each waits ~2.5 us
-// on its loads, and a grouped launch also queues a work group per group the
-// routing could make (at 32 tokens x top-8 over 128 experts: 144 possible,
-// ~45 made).  Here one work group per CU walks (group, run of row tiles)
-// items, sized on the device from the groups actually made, and streams each
-// tile's weights through a ring of three LDS stages with direct
-// global->LDS loads (16 bytes per lane, 1 KB of LDS per wave instruction):
-// the next tiles load while one computes, and the registers hold only the
-// group's activations.
-//
-// Geometry: a tile is TR = 16*RG rows x all NB super-blocks of one matrix
-// (both for the fused gate/up); wave (rg, b) computes block b of rows
-// 16*rg .. +16, RG = 8 / NB.  LDS slot j of a matrix is (block, 16-byte chunk
-// c, row r), r fastest, so a wave's operand read is 1 KB of consecutive
-// slots and a row header a broadcast; chunk 0 of a (row, block) is its
-// header, 1..8 its quants.
-template <bool FUSED, int NB>
-struct Mmqs {
-    static constexpr int RG = 8 / NB, W = RG * NB, TR = 16 * RG;
-    static constexpr int MAT = TR * NB * 9; // 16-byte chunks per matrix
-    static constexpr int MATS = FUSED ? 2 : 1;
-    static constexpr int CH = MATS * MAT;
-    static constexpr int INS = (CH + 63) / 64; // 1 KB wave loads per tile, dealt round robin:
-    static constexpr int K = (INS + W - 1) / W; // waves below KW issue K, the rest K - 1
-    static constexpr int KW = INS % W == 0 ? W : INS % W;
-    static constexpr int STAGE = INS * 1024;    // bytes per stage
-    static constexpr int RS = q4kv_rs(TR);
-    static constexpr int PART = MATS * NB * 16 * RS; // floats
-    static constexpr size_t LDS = 3 * (size_t)STAGE + 2 * 4 * (size_t)PART;
-    static_assert(LDS <= 160 * 1024, "three stages and two sums buffers fit a CU's LDS");
-};
-
-// Global address of chunk j of a tile (rows row0 .. +TR, clamped to the
-// matrix) of the Q4_K matrix at mb.
-template <int NB, int TR>
-__device__ __forceinline__ const uint8_t *mmqs_chunk(const uint8_t *mb, int rows, int row0, int j) {
-    const int bb = j / (9 * TR), c = (j / TR) % 9, r = j % TR;
-    const int row = min(row0 + r, rows - 1);
-    return mb + ((size_t)row * NB + bb) * 144 + c * 16;
-}
-
-// A work-group barrier that waits for this wave's LDS stores only: the
-// workgroup fence of lds_barrier also waits for the direct-to-LDS loads in
-// flight (they are LDS stores), which would drain the ring at every tile.
-// The loads a barrier must cover are waited for explicitly (wait_vm) before
-// it; the asm's memory clobber keeps the compiler from moving LDS accesses
-// across it.
-__device__ __forceinline__ void ring_barrier() {
-    __builtin_amdgcn_s_waitcnt(0xC07F); // lgkmcnt(0); vmcnt and expcnt left open
-    asm volatile("s_barrier" ::: "memory");
-}
-
-// Reads of a stage.  The compiler cannot tell the three stages apart, so
-// before any LDS read it would wait for every direct-to-LDS load in flight;
-// the reads are issued as one asm block instead, ending in its own lgkmcnt
-// wait, after the explicit vmcnt wait and barrier that order them behind
-// their own tile's loads.
-typedef unsigned mmqs_u4 __attribute__((ext_vector_type(4)));
-__device__ __forceinline__ uint32_t lds_off(const void *p) {
-    return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void *)p;
-}
-__device__ __forceinline__ void lds_read3(uint32_t a0, uint32_t a1, uint32_t a2, uint4 &r0, uint4 &r1, uint4 &r2) {
-    mmqs_u4 x0, x1, x2;
-    asm volatile("ds_read_b128 %0, %3\n\tds_read_b128 %1, %4\n\tds_read_b128 %2, %5\n\ts_waitcnt lgkmcnt(0)"
-                 : "=&v"(x0), "=&v"(x1), "=&v"(x2)
-                 : "v"(a0), "v"(a1), "v"(a2)
-                 : "memory");
-    r0 = make_uint4(x0.x, x0.y, x0.z, x0.w);
-    r1 = make_uint4(x1.x, x1.y, x1.z, x1.w);
-    r2 = make_uint4(x2.x, x2.y, x2.z, x2.w);
-}
-
-template <int N>
-__device__ __forceinline__ void wait_vm() { // s_waitcnt vmcnt(N) alone
-    static_assert(N >= 0 && N < 64, "vmcnt");
-    __builtin_amdgcn_s_waitcnt(0x0F70 | (N & 15) | ((N >> 4) << 14));
-}
-
-template <bool FUSED, int NB>
-__global__ __launch_bounds__(64 * MMQ_WAVES) void mmqs_kernel(DmmvParams p) {
-    using G = Mmqs<FUSED, NB>;
-    constexpr int TOK = 16, TR = G::TR, RS = G::RS, K = G::K;
-    constexpr int TPS = 8, NS = TOK / TPS; // tokens per MFMA set (x 2 groups = 16 A rows), sets
-    __shared__ __align__(16) uint8_t st0[G::STAGE], st1[G::STAGE], st2[G::STAGE];
-    __shared__ __align__(16) float part0[G::PART], part1[G::PART];
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), ln = threadIdx.x & 63;
-    const int r16 = ln & 15, q4 = ln >> 4;
-    const int rg = wave % G::RG, b = wave / G::RG;
-    const int rl = 16 * rg + r16;
-    const int tiles = (p.rows + TR - 1) / TR;
-    const size_t mat = (size_t)NB * TOK * RS;
-    const mmq_i4 z = {0, 0, 0, 0};
-    const bool live = (q4 >> 1) == (r16 & 1); // A row r16 = (token r16/2, group part r16&1)
-    // items: each group's tiles in cpg runs, so that the items about fill the grid
-    const int ng = p.n_groups_dev ? *p.n_groups_dev : p.n_groups;
-    const int nwg = gridDim.x;
-    const int cpg = ng > 0 ? max(1, min(tiles, nwg / ng)) : 1;
-    const int run = (tiles + cpg - 1) / cpg;
-    const int items = ng * cpg;
-    for (int item = blockIdx.x; item < items; item += nwg) {
-        const int gi = item / cpg, t0 = (item % cpg) * run;
-        const int nt = min(run, tiles - t0);
-        if (nt <= 0)
-            continue;
-        const DmmvGroup grp = p.groups[gi];
-        const int n = grp.n, ns = (n + TPS - 1) / TPS;
-        const uint8_t *pb = p.w + (size_t)grp.plane * p.plane_bytes;
-        const uint8_t *pb2 = FUSED ? p.w2 + (size_t)grp.plane * p.plane_bytes : pb;
-        // the group's activations as A rows, and the block scales of this
-        // lane's result tokens 2*q4 + jj of each set
-        auto vec_of = [&](int t) {
-            if (p.group_src)
-                return p.group_src[(size_t)gi * p.group_stride + t];
-            t = min(t, n - 1);
-            return p.pos_ident ? grp.first + t : p.pair_src[grp.first + t];
-        };
-        mmq_i4 xa[NS][4];
-        float xd[NS][2];
+    const int row = row0 + r16;
+    if (row >= p.rows)
+        return;
+    auto put = [&](int t, float v) {
+        if (t >= n)
+            return;
+        const int dst = ident || p.pos_ident ? grp.first + t : p.pair_dst[grp.first + t];
+        float *o = p.out + (size_t)dst * p.out_stride + row;
+        *o = p.accumulate ? *o + v : v;
+    };
+    if constexpr (K4) {
 #pragma unroll
-        for (int s = 0; s < NS; s++) {
-            const int8_t *xr = p.xq + (size_t)vec_of(TPS * s + r16 / 2) * p.cols + 256 * b;
-#pragma unroll
-            for (int j = 0; j < 4; j++)
-                xa[s][j] = live && s < ns ? *(const mmq_i4 *)(xr + q4kv_xoff(j, q4)) : z;
+        for (int s = 0; s < 2; s++)
 #pragma unroll
             for (int jj = 0; jj < 2; jj++)
-                xd[s][jj] = s < ns ? p.xd[(size_t)vec_of(TPS * s + 2 * q4 + jj) * NB + b] : 0.0f;
-        }
-        // one tile's weights into a stage: this wave's 1 KB pieces I = wave + W*i
-        auto issue = [&](int tile, uint8_t *stg) {
-            const int row0 = tile * TR;
+                put(8 * s + 2 * q4 + jj, FUSED ? swiglu1(acc4[0][s][jj], acc4[M - 1][s][jj]) : acc4[0][s][jj]);
+    } else {
 #pragma unroll
-            for (int i = 0; i < K; i++) {
-                const int I = wave + G::W * i;
-                if (I >= G::INS)
-                    break; // (uniform)
-                int j = I * 64 + ln;
-                const uint8_t *src = pb; // past the tile's chunks: a valid address, never read back
-                if (j < G::CH) {
-                    const uint8_t *mb = pb;
-                    if (FUSED && j >= G::MAT) {
-                        mb = pb2;
-                        j -= G::MAT;
-                    }
-                    src = mmqs_chunk<NB, TR>(mb, p.rows, row0, j);
-                }
-                __builtin_amdgcn_global_load_lds((const void *)src,
-                                                 (__attribute__((address_space(3))) void *)(stg + I * 1024), 16, 0, 0);
-            }
-        };
-        // tile k's loads have landed once only the next tile's (this wave's
-        // K or K - 1 pieces, issued after it) may be outstanding
-        auto wait_tile = [&](int k) {
-            if (k + 1 >= nt)
-                wait_vm<0>();
-            else if (wave < G::KW)
-                wait_vm<K>();
-            else
-                wait_vm<K - 1>();
-        };
-        // a tile's MFMAs from its stage, its per-block values into pbuf
-        auto compute = [&](const uint8_t *stg, float *pbuf) {
-            auto frag = [&](int m) {
-                const uint32_t mbase = lds_off(stg) + (uint32_t)m * G::MAT * 16;
-                Q4kTileV w;
-                lds_read3(mbase + ((b * 9 + 0) * TR + rl) * 16, mbase + ((b * 9 + 1 + q4) * TR + rl) * 16,
-                          mbase + ((b * 9 + 5 + q4) * TR + rl) * 16, w.hdr, w.qs[0], w.qs[1]);
-                return w;
-            };
-            float r[NS][2], r2[NS][2];
-            q4kv_tile<NS>(frag(0), q4, ns, xa, xd, r);
-            if constexpr (FUSED)
-                q4kv_tile<NS>(frag(1), q4, ns, xa, xd, r2);
+        for (int mt = 0; mt < MT; mt++)
 #pragma unroll
-            for (int s = 0; s < NS; s++)
-                if (s < ns)
-#pragma unroll
-                    for (int jj = 0; jj < 2; jj++) {
-                        const size_t o = ((size_t)b * TOK + TPS * s + 2 * q4 + jj) * RS + rl;
-                        pbuf[o] = r[s][jj];
-                        if constexpr (FUSED)
-                            pbuf[mat + o] = r2[s][jj];
-                    }
-        };
-        // tile k's outputs: every (token, row) summed over its blocks in block
-        // order from pbuf (all the block values read first), SwiGLU(gate, up)
-        // when fused, stored -- pos_ident, no residual add (launch_mmqs), so
-        // no global load here, which would wait (vmcnt counts in order) for
-        // the tiles in flight
-        auto reduce = [&](int k, const float *pbuf) {
-            const int row0 = (t0 + k) * TR;
-            for (int idx = threadIdx.x; idx < n * TR; idx += blockDim.x) {
-                const int tk = idx / TR, rr = idx % TR;
-                if (row0 + rr >= p.rows)
-                    continue;
-                const float *pv = pbuf + (size_t)tk * RS + rr;
-                float v1[NB], v2[NB];
-#pragma unroll
-                for (int bb = 0; bb < NB; bb++) {
-                    v1[bb] = pv[(size_t)bb * TOK * RS];
-                    if constexpr (FUSED)
-                        v2[bb] = pv[mat + (size_t)bb * TOK * RS];
-                }
-                float acc = 0.0f;
-#pragma unroll
-                for (int bb = 0; bb < NB; bb++)
-                    acc = acc + v1[bb];
-                float v = acc;
-                if constexpr (FUSED) {
-                    float acc2 = 0.0f;
-#pragma unroll
-                    for (int bb = 0; bb < NB; bb++)
-                        acc2 = acc2 + v2[bb];
-                    v = swiglu1(acc, acc2);
-                }
-                p.out[(size_t)(grp.first + tk) * p.out_stride + row0 + rr] = v;
-            }
-        };
-        // Step k: wait for tile k, one barrier, then tile k - 1's sums out (its
-        // values were written before this barrier), tile k + 2's loads into
-        // the stage tile k - 1 computed from (every wave has passed its reads),
-        // and tile k's MFMAs.  The sums buffers alternate, so tile k's values
-        // are written while tile k - 1's are read.  The stores precede the next
-        // loads, so the next wait (vmcnt counts in order) covers them too.
-        auto step = [&](int k, const uint8_t *cur, uint8_t *refill) {
-            wait_tile(k);
-            ring_barrier();
-            if (k > 0)
-                reduce(k - 1, (k - 1) & 1 ? part1 : part0);
-            if (k + 2 < nt)
-                issue(t0 + k + 2, refill);
-            compute(cur, k & 1 ? part1 : part0);
-        };
-        issue(t0, st0);
-        if (nt > 1)
-            issue(t0 + 1, st1);
-        for (int k = 0; k < nt; k += 3) {
-            step(k, st0, st2);
-            if (k + 1 >= nt)
-                break;
-            step(k + 1, st1, st0);
-            if (k + 2 >= nt)
-                break;
-            step(k + 2, st2, st1);
-        }
-        ring_barrier();
-        reduce(nt - 1, (nt - 1) & 1 ? part1 : part0);
-        ring_barrier(); // the next item's stages and sums reuse this one's LDS
+            for (int i = 0; i < 4; i++)
+                put(16 * mt + 4 * q4 + i, acc6[mt][i]);
     }
 }
 
-// The streamed launch: the fused gate/up of grouped experts (not lane
-// groups), Q4_K over 2048 columns, up to 16 tokens per group, outputs at the
-// pair positions with no residual add; false = not served.
-static bool launch_mmqs(int t, bool fused, const DmmvParams &p, hipStream_t st) {
-    if (t != LH_Q4_K || !fused || p.ident_n > 0 || !p.groups || !p.pos_ident || p.accumulate || p.rows < 1 ||
-        p.cols != 8 * 256)
+// Waves per SIMD of each form, as its registers allow (3: 168, 2: 256, 4: 128).
+template <int T, int MT, bool FUSED, bool XL> constexpr int mmw_occ() {
+    return XL ? (FUSED || MT == 2 ? 3 : 4) : (FUSED || MT == 2 ? 2 : 3);
+}
+template <int T, int MT, bool FUSED>
+static void mmw_launch_t(const DmmvParams &p, hipStream_t st) {
+    const int groups = p.ident_n > 0 ? (p.ident_n + 16 * MT - 1) / (16 * MT) : p.n_groups;
+    const int tiles = (p.rows + 15) / 16;
+    const dim3 grid((tiles + MMW_W - 1) / MMW_W, groups), block(64 * MMW_W);
+    if (p.cols <= MMW_XL_COLS)
+        hipLaunchKernelGGL((mmw_kernel<T, MT, FUSED, true, mmw_occ<T, MT, FUSED, true>()>), grid, block,
+                           (mmw_lds<T, MT, true>(p.cols)), st, p);
+    else
+        hipLaunchKernelGGL((mmw_kernel<T, MT, FUSED, false, mmw_occ<T, MT, FUSED, false>()>), grid, block,
+                           (mmw_lds<T, MT, false>(p.cols)), st, p);
+}
+
+// Which launches mmw_kernel takes from the one-shot kernel: every grouped
+// (expert) one, and lane groups from MMW_MIN_WAVES (row tile, 16 lanes) pairs,
+// below which too few waves stream (measured, us per launch, one-shot / mmw:
+// Q4_K 8192 x 4096 at 16 lanes, 512 pairs, 14.4 / 15.1; at 32 lanes, 1024,
+// 22.6 / 15.8; Q6_K 16384 x 4096 at 16 lanes, 1024, 32.7 / 20.6).  Its byte
+// offsets are 32-bit.
+constexpr long MMW_MIN_WAVES = 1024;
+static bool mmw_serves(int t, const DmmvParams &p) {
+    const long tiles = (p.rows + 15) / 16;
+    if ((size_t)p.rows * (p.cols / 256) * block_bytes(t) >= ((size_t)1 << 32))
         return false;
-    static int cus = 0;
-    if (cus == 0) {
-        int dev = 0, c = 0;
-        if (hipGetDevice(&dev) == hipSuccess &&
-            hipDeviceGetAttribute(&c, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && c > 0)
-            cus = c;
-        else
-            cus = 256;
-    }
-    // one work group per CU (its LDS fills one)
-    hipLaunchKernelGGL((mmqs_kernel<true, 8>), dim3(cus), dim3(64 * Mmqs<true, 8>::W), 0, st, p);
-    return true;
+    return p.ident_n <= 0 || tiles * ((p.ident_n + 15) / 16) >= MMW_MIN_WAVES;
 }
-
 
 // Shape of a launch: KS = min(nb, MMQ_WAVES) slices of SBW super-blocks per
 // wave, as many row tiles beside them as fit the wave count and 64 KB of LDS,
@@ -1078,31 +1170,11 @@ bool mmq_supported(int t, int cols, int max_tok, bool fused) {
     return mmq_shape(16, cols, (max_tok + 15) / 16, fused, rg, ks, sbw);
 }
 
-// Streaming serves the lane-group (identity) launches with at least
-// MMQ_STREAM_MIN (row tile, group) pairs (the head): for the grouped expert
-// launches the one-shot kernel measured faster (its groups already give
-// thousands of short work groups).  Its two register sets hold one work
-// group per CU, so the pairs are split over about MMQ_STREAM_WGS work groups
-// (one per CU, no partial second round), at most MMQ_MAX_NTILE tiles each.
-constexpr int MMQ_STREAM_MIN = 1024;
-constexpr int MMQ_STREAM_WGS = 256;
-constexpr int MMQ_MAX_NTILE = 64;
-
 template <int T, int MT, bool FUSED>
 static void mmq_launch_t(const DmmvParams &p, int rg, int ks, int sbw, hipStream_t st) {
     const size_t lds = mmq_lds_bytes(p.cols, MT, rg, FUSED);
     const int groups = p.ident_n > 0 ? (p.ident_n + 16 * MT - 1) / (16 * MT) : p.n_groups;
     const int tiles = (p.rows + 16 * rg - 1) / (16 * rg);
-    if (sbw == 1 && p.ident_n > 0 && 2 * lds <= 64 * 1024) {
-        const long pairs = (long)tiles * groups;
-        int ntile = pairs < MMQ_STREAM_MIN ? 1 : (int)((pairs + MMQ_STREAM_WGS - 1) / MMQ_STREAM_WGS);
-        ntile = ntile > MMQ_MAX_NTILE ? MMQ_MAX_NTILE : ntile;
-        if (ntile > 1) {
-            const dim3 grid((tiles + ntile - 1) / ntile, groups), block(64 * rg * ks);
-            hipLaunchKernelGGL((mmq_stream_kernel<T, MT, FUSED>), grid, block, 2 * lds, st, p, rg, ntile);
-            return;
-        }
-    }
     const dim3 grid(tiles, groups), block(64 * rg * ks);
     if (sbw == 1)
         hipLaunchKernelGGL((mmq_kernel<T, MT, FUSED, 1>), grid, block, lds, st, p, rg, ks);
@@ -1158,13 +1230,19 @@ bool launch_mmq(int t, int max_tok, bool fused, const DmmvParams &p, hipStream_t
         return true;
     }
     const int mt = max_tok > 16 ? 2 : 1;
-    int rg, ks, sbw;
-    if (!mmq_shape(p.rows, p.cols, mt, fused, rg, ks, sbw))
-        return false;
-    if (mt == 1 && launch_mmqs(t, fused, p, st)) {
+    if (mmw_serves(t, p)) {
+        if (t == LH_Q4_K)
+            fused ? mmw_launch_t<LH_Q4_K, 1, true>(p, st) : mmw_launch_t<LH_Q4_K, 1, false>(p, st);
+        else if (mt == 1)
+            mmw_launch_t<LH_Q6_K, 1, false>(p, st);
+        else
+            mmw_launch_t<LH_Q6_K, 2, false>(p, st);
         note_launch();
         return true;
     }
+    int rg, ks, sbw;
+    if (!mmq_shape(p.rows, p.cols, mt, fused, rg, ks, sbw))
+        return false;
     if (t == LH_Q4_K) {
         if (mt == 1)
             fused ? mmq_launch_t<LH_Q4_K, 1, true>(p, rg, ks, sbw, st)
