@@ -1435,11 +1435,13 @@ int frame_layer(const FrameCall &c, const loomhip_layer &l, size_t li, uint32_t 
     p.n_groups = w.n_groups;
     p.out = w.act;
     p.out_stride = (int)l.ffn;
-    p.rpw = dmmv_pick_rpw(l.ffn_gate_t, D.dim, (int)l.ffn, w.n_groups, w.nt, true);
-    if (!launch_dmmv(l.ffn_gate_t, w.nt, true, p, st))
+    const bool mq = use_mmq(l.ffn_gate_t, D.dim, (int)n, 16, true);
+    p.ident_n = mq ? (int)n : 0;
+    p.rpw = mq ? 0 : dmmv_pick_rpw(l.ffn_gate_t, D.dim, (int)l.ffn, w.n_groups, w.nt, true);
+    if (!(mq ? launch_mmq(l.ffn_gate_t, 16, true, p, st) : launch_dmmv(l.ffn_gate_t, w.nt, true, p, st)))
         return fail(LOOMHIP_ERR_ARG, "token_frame: gate/up matvec declined");
     launch_quant_act(l.ffn_down_t, w.act, (int)l.ffn, (int)l.ffn, (int)n, w.qa_ffn, st);
-    if (!frame_matvec(l.ffn_down_t, l.ffn_down, D.dim, (int)l.ffn, w, n, w.qa_ffn, w.x, 1, st))
+    if (!frame_matvec(l.ffn_down_t, l.ffn_down, D.dim, (int)l.ffn, w, n, w.qa_ffn, w.x, 1, st, LOOMHIP_KT_DENSE, true))
         return fail(LOOMHIP_ERR_ARG, "token_frame: down matvec declined");
     return LOOMHIP_OK;
 }

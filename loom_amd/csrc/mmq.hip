@@ -942,17 +942,20 @@ static void mmw_launch_t(const DmmvParams &p, hipStream_t st) {
 }
 
 // Which launches mmw_kernel takes from the one-shot kernel: every grouped
-// (expert) one, and lane groups from MMW_MIN_WAVES (row tile, 16 lanes) pairs,
-// below which too few waves stream (measured, us per launch, one-shot / mmw:
-// Q4_K 8192 x 4096 at 16 lanes, 512 pairs, 14.4 / 15.1; at 32 lanes, 1024,
-// 22.6 / 15.8; Q6_K 16384 x 4096 at 16 lanes, 1024, 32.7 / 20.6).  Its byte
-// offsets are 32-bit.
-constexpr long MMW_MIN_WAVES = 1024;
-static bool mmw_serves(int t, const DmmvParams &p) {
+// (expert) one, and lane groups from MMW_MIN_WAVES (row tile, 16 lanes) pairs
+// (512 for a fused pair, twice the bytes per wave), below which too few waves
+// stream.  Measured, us per launch, one-shot / mmw: Q4_K 8192 x 4096 at 16
+// lanes (512 pairs) 14.4 / 15.1, at 32 (1024) 22.6 / 15.8; 7168 x 2048 at 24
+// (896) 13.1 / 9.8; Q6_K 16384 x 4096 at 16 (1024) 32.7 / 20.6; fused 2048 x
+// 7168 at 24 (256) 25.6 / 32.1, at 64 (512) 44.8 / 32.6; fused 4096 x 2048
+// at 24 (512) 12.7 / 13.2, at 64 (1024) 20.4 / 14.0.  Its byte offsets are
+// 32-bit.
+constexpr long MMW_MIN_WAVES = 768, MMW_MIN_WAVES_FUSED = 512;
+static bool mmw_serves(int t, bool fused, const DmmvParams &p) {
     const long tiles = (p.rows + 15) / 16;
     if ((size_t)p.rows * (p.cols / 256) * block_bytes(t) >= ((size_t)1 << 32))
         return false;
-    return p.ident_n <= 0 || tiles * ((p.ident_n + 15) / 16) >= MMW_MIN_WAVES;
+    return p.ident_n <= 0 || tiles * ((p.ident_n + 15) / 16) >= (fused ? MMW_MIN_WAVES_FUSED : MMW_MIN_WAVES);
 }
 
 // Shape of a launch: KS = min(nb, MMQ_WAVES) slices of SBW super-blocks per
@@ -1230,7 +1233,7 @@ bool launch_mmq(int t, int max_tok, bool fused, const DmmvParams &p, hipStream_t
         return true;
     }
     const int mt = max_tok > 16 ? 2 : 1;
-    if (mmw_serves(t, p)) {
+    if (mmw_serves(t, fused, p)) {
         if (t == LH_Q4_K)
             fused ? mmw_launch_t<LH_Q4_K, 1, true>(p, st) : mmw_launch_t<LH_Q4_K, 1, false>(p, st);
         else if (mt == 1)

@@ -116,8 +116,12 @@ int dense_ffn_add(const DenseFfn &f, const float *x, size_t n, size_t dim, float
     p.n_groups = ng;
     p.out = act;
     p.out_stride = (int)f.ffn;
-    p.rpw = dmmv_pick_rpw(f.gate_t, (int)dim, (int)f.ffn, ng, nt, true);
-    if (!launch_dmmv(f.gate_t, nt, true, p, st))
+    // from MMQ_MIN_TOK tokens each matmul runs on the matrix cores where its type and shape are
+    // served (7168 -> 2048 -> 7168 Q4_K at 24 tokens: gate/up 48 -> 25 us, down 33 -> 10 us)
+    const bool mq = use_mmq(f.gate_t, (int)dim, (int)n, 16, true);
+    p.ident_n = mq ? (int)n : 0;
+    p.rpw = mq ? 0 : dmmv_pick_rpw(f.gate_t, (int)dim, (int)f.ffn, ng, nt, true);
+    if (!(mq ? launch_mmq(f.gate_t, 16, true, p, st) : launch_dmmv(f.gate_t, nt, true, p, st)))
         return fail(LOOMHIP_ERR_ARG, "shared expert: gate/up partials exceed LDS");
     launch_quant_act(f.down_t, act, (int)f.ffn, (int)f.ffn, (int)n, qa, st);
     DmmvParams d{};
@@ -134,8 +138,10 @@ int dense_ffn_add(const DenseFfn &f, const float *x, size_t n, size_t dim, float
     d.out = out;
     d.out_stride = (int)dim;
     d.accumulate = add ? 1 : 0; // add: out = out + value
-    d.rpw = dmmv_pick_rpw(f.down_t, (int)f.ffn, (int)dim, ng, nt, false);
-    if (!launch_dmmv(f.down_t, nt, false, d, st))
+    const bool mqd = use_mmq(f.down_t, (int)f.ffn, (int)n, 32, false);
+    d.ident_n = mqd ? (int)n : 0;
+    d.rpw = mqd ? 0 : dmmv_pick_rpw(f.down_t, (int)f.ffn, (int)dim, ng, nt, false);
+    if (!(mqd ? launch_mmq(f.down_t, 32, false, d, st) : launch_dmmv(f.down_t, nt, false, d, st)))
         return fail(LOOMHIP_ERR_ARG, "shared expert: down partials exceed LDS");
     return LOOMHIP_OK;
 }

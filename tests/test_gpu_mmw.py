@@ -66,3 +66,24 @@ def test_streamed_matmul_extreme_integers(be, oracle, t):
     xs[1::2] = -3.0
     xs[2::4, ::2] = -1.0
     _check(be, oracle, t, raw, xs, rows, cols)
+
+
+@pytest.mark.parametrize("n", [16, 33])
+def test_dense_ffn_frame_on_matrix_cores(oracle, n):
+    """A llama-architecture model in Q4_K / Q6_K: from 16 lanes its dense
+    FFN's gate/up and down run on the matrix cores (frame_layer).  PARITY
+    per-lane logits bit-identical to lo_decode_batch on identical state."""
+    import dataclasses
+
+    import loom_amd
+    from loom_amd import frame as lh
+    from oracle.model import OracleModel
+    from test_gpu_frame import _batch_steps
+
+    loom_amd.init(0)
+    spec = dataclasses.replace(lh.stories15m(ctx_len=96), dim=512, n_layers=2, vocab=1024, n_heads=8, n_kv_heads=4,
+                               head_dim=64, rope_dim=64, ffn=1280, embed_t=Q4_K, output_t=Q6_K, wq_t=Q4_K, wk_t=Q4_K,
+                               wv_t=Q6_K, wo_t=Q4_K, ffn_gate_t=Q4_K, ffn_down_t=Q6_K)
+    dm = lh.DeviceModel.synth(spec, seed=17, keep_ggml=True)
+    rels, same = _batch_steps(lh, OracleModel(oracle, dm), dm, n, 2, 60, seed=n)
+    assert rels.max() == 0.0 and same
