@@ -1113,8 +1113,8 @@ static FrameWs frame_layout(char *base, size_t n, const loomhip_model *m, size_t
     return w;
 }
 
-// mmq_ok: the matrix cores from MMQ_MIN_TOK lanes on, in groups of mmq_group
-// lanes (16 for wo: more work groups for its 2048 rows; 32 for the head,
+// mmq_ok: the matrix cores where mmq_dense takes the lanes, in groups of
+// mmq_group (16 for wo: more work groups for its 2048 rows; 32 for the head,
 // whose 255 MB would be read once per group).
 static bool frame_matvec(int t, const void *wt, int rows, int cols, const FrameWs &w, size_t n,
                          QAct x, float *out, int accumulate, hipStream_t st, int tag = LOOMHIP_KT_DENSE,
@@ -1134,15 +1134,19 @@ static bool frame_matvec(int t, const void *wt, int rows, int cols, const FrameW
     p.out = out;
     p.out_stride = rows;
     p.accumulate = accumulate;
-    const bool mq = mmq_ok && use_mmq(t, cols, (int)n, 32, false);
+    const bool mq = mmq_ok && mmq_dense(t, rows, cols, (int)n, false);
     if (mq)
         p.ident_n = (int)n;
     p.rpw = mq ? 0 : dmmv_pick_rpw(t, cols, rows, w.n_groups, w.nt, false);
     const int ph = prof_begin(tag, st);
-    const bool ok = mq ? launch_mmq(t, mmq_group, false, p, st) : launch_dmmv(t, w.nt, false, p, st);
+    const bool ok = mq ? launch_mmq(t, n > 16 ? mmq_group : 16, false, p, st) : launch_dmmv(t, w.nt, false, p, st);
     prof_end(ph, st);
     return ok;
 }
+
+// us per two-layer step (Qwen3-30B-A3B shapes), dot4 / matrix-core q, k, v: 5 lanes 336.6 / 332.9,
+// 15 lanes 349.5 / 332.7
+constexpr size_t QKV_MMQ_MIN = 5;
 
 // q, k and v of one layer against the normalised input, one launch.  With
 // fused: one lane in PARITY, the launch normalises x itself (the exact sum)
@@ -1173,10 +1177,9 @@ static bool frame_qkv(const loomhip_layer &l, const FrameDims &D, const FrameWs 
         prof_end(ph, st);
         return *fused;
     }
-    // from MMQ_MIN_TOK lanes: the matrix cores, the three matrices in one
+    // from QKV_MMQ_MIN lanes: the matrix cores, the three matrices in one
     // launch, lanes in groups of 16
-    if (use_mmq(l.wq_t, D.dim, (int)n, 32, false) && use_mmq(l.wk_t, D.dim, (int)n, 32, false) &&
-        use_mmq(l.wv_t, D.dim, (int)n, 32, false)) {
+    if (n >= QKV_MMQ_MIN) {
         DmmvSegParams mp = sp;
         mp.base.ident_n = (int)n;
         const int ph = prof_begin(LOOMHIP_KT_QKV, st);
@@ -1435,7 +1438,7 @@ int frame_layer(const FrameCall &c, const loomhip_layer &l, size_t li, uint32_t 
     p.n_groups = w.n_groups;
     p.out = w.act;
     p.out_stride = (int)l.ffn;
-    const bool mq = use_mmq(l.ffn_gate_t, D.dim, (int)n, 16, true);
+    const bool mq = mmq_dense(l.ffn_gate_t, (int)l.ffn, D.dim, (int)n, true);
     p.ident_n = mq ? (int)n : 0;
     p.rpw = mq ? 0 : dmmv_pick_rpw(l.ffn_gate_t, D.dim, (int)l.ffn, w.n_groups, w.nt, true);
     if (!(mq ? launch_mmq(l.ffn_gate_t, 16, true, p, st) : launch_dmmv(l.ffn_gate_t, w.nt, true, p, st)))

@@ -86,10 +86,13 @@ void launch_synth(int t, void *dst, size_t rows, size_t cols, size_t planes, uin
 bool dmmv_supported(int t, int cols);
 // Returns false (launching nothing) when the partials would not fit in LDS.
 bool launch_dmmv(int t, int nt, bool fused, const DmmvParams &p, hipStream_t st);
-// Matrix-core variant for Q4_K / Q6_K with groups of up to max_tok (<= 32)
-// tokens: the same results bit for bit.  False (nothing launched) when the
-// type or the LDS need is not served.
-bool mmq_supported(int t, int cols, int max_tok, bool fused);
+// Matrix-core variant, the same results bit for bit.  mmq_dense: whether it
+// takes n vectors against one matrix (a fused pair) from the dot4 matvec;
+// mmq_experts: whether it takes the expert matmuls of n tokens, in groups of
+// up to 16.  launch_mmq: groups of up to max_tok (<= 32) tokens; false
+// (nothing launched) for a type or shape it does not serve.
+bool mmq_dense(int t, int rows, int cols, int n, bool fused);
+bool mmq_experts(int gate_t, int down_t, int dim, int ffn, int n);
 bool launch_mmq(int t, int max_tok, bool fused, const DmmvParams &p, hipStream_t st);
 bool launch_mmq_seg(DmmvSegParams sp, hipStream_t st);
 // Rows per wave chosen for a launch of `rows` rows x `groups` groups.

@@ -941,23 +941,6 @@ static void mmw_launch_t(const DmmvParams &p, hipStream_t st) {
                            (mmw_lds<T, MT, false>(p.cols)), st, p);
 }
 
-// Which launches mmw_kernel takes from the one-shot kernel: every grouped
-// (expert) one, and lane groups from MMW_MIN_WAVES (row tile, 16 lanes) pairs
-// (512 for a fused pair, twice the bytes per wave), below which too few waves
-// stream.  Measured, us per launch, one-shot / mmw: Q4_K 8192 x 4096 at 16
-// lanes (512 pairs) 14.4 / 15.1, at 32 (1024) 22.6 / 15.8; 7168 x 2048 at 24
-// (896) 13.1 / 9.8; Q6_K 16384 x 4096 at 16 (1024) 32.7 / 20.6; fused 2048 x
-// 7168 at 24 (256) 25.6 / 32.1, at 64 (512) 44.8 / 32.6; fused 4096 x 2048
-// at 24 (512) 12.7 / 13.2, at 64 (1024) 20.4 / 14.0.  Its byte offsets are
-// 32-bit.
-constexpr long MMW_MIN_WAVES = 768, MMW_MIN_WAVES_FUSED = 512;
-static bool mmw_serves(int t, bool fused, const DmmvParams &p) {
-    const long tiles = (p.rows + 15) / 16;
-    if ((size_t)p.rows * (p.cols / 256) * block_bytes(t) >= ((size_t)1 << 32))
-        return false;
-    return p.ident_n <= 0 || tiles * ((p.ident_n + 15) / 16) >= (fused ? MMW_MIN_WAVES_FUSED : MMW_MIN_WAVES);
-}
-
 // Shape of a launch: KS = min(nb, MMQ_WAVES) slices of SBW super-blocks per
 // wave, as many row tiles beside them as fit the wave count and 64 KB of LDS,
 // but no more than the matrix has.
@@ -1162,15 +1145,413 @@ static bool launch_mmq32(int t, int max_tok, const DmmvParams &p, hipStream_t st
     return true;
 }
 
-bool mmq_supported(int t, int cols, int max_tok, bool fused) {
-    if (t == LH_Q8_0 || t == LH_Q4_0)
+// ---- Q8_0 / Q4_0 streamed in block order ------------------------------------------
+// mmw_kernel's shape for 32-value blocks: a wave owns 16 rows for up to 16
+// tokens of a group and walks them in units of 8 blocks (256 columns),
+// weights loaded in address order and turned through its LDS, two units in
+// registers or in flight.  A 64-deep MFMA spans two blocks; its A rows are
+// (token, block) pairs (8 tokens a set, zeros on the other block's quarters),
+// so one MFMA over the unmasked weights gives both blocks' integer dots of 8
+// tokens, and the tails (d * xd) * f32(isum) add in block order.  Q4_0's
+// weights enter as nibble - 8, the reference's sum q*x - 8*sum x as one exact
+// integer.  Bound by the weights' bytes at few tokens and by the four VALU
+// operations of each (token, row, block)'s tail at 16.
+// Measured (us per launch, events; dot4 / this): experts 2048 -> 768 fused
+// over 64 planes at 4 tokens each Q4_0 65 / 33, Q8_0 76 / 72, at 10 182 / 38
+// and 185 / 87; 768 -> 2048 at 10 57 / 22 and 92 / 29; 11008 x 4096 Q8_0 at
+// 32 vectors 126 / 31.
+template <int T> struct Mmw32Blk {
+    static constexpr bool Q8 = T == LH_Q8_0;
+    static constexpr int QB = Q8 ? 32 : 16;          // quant bytes per block
+    static constexpr int CH = Q8 ? 16 : 8;           // 16-byte chunks per row and unit
+    static constexpr int NL = Q8 ? 4 : 2;            // loads: 64 / CH rows each
+    static constexpr int ROWB = 16 * CH + 16;        // odd chunk stride in LDS
+    static constexpr int BYTES = 16 * ROWB + 256;    // then the scales, f16 [row][8]
+    mmq_i4 v[NL];
+    uint32_t d0, d1; // blocks 2 * (ln & 3), + 1 of row ln / 4
+    struct Src {
+        const uint8_t *q, *d;
+        uint32_t row[NL], drow; // byte offset of the lane's row per load; block index of row ln / 4
+    };
+    __device__ __forceinline__ static Src src(const uint8_t *wb, int rows, int nb, int row0, int ln) {
+        Src s;
+        s.q = wb;
+        s.d = wb + (size_t)rows * nb * QB;
+#pragma unroll
+        for (int i = 0; i < NL; i++)
+            s.row[i] = (uint32_t)min(row0 + (64 / CH) * i + ln / CH, rows - 1) * (uint32_t)(nb * QB);
+        s.drow = (uint32_t)min(row0 + (ln >> 2), rows - 1) * (uint32_t)nb;
+        return s;
+    }
+    // unit u: chunks and blocks past the row's end read its last ones
+    __device__ __forceinline__ void load(const Src &s, int u, int nb, int ln) {
+        const uint32_t c = 16u * (uint32_t)min(CH * u + ln % CH, nb * QB / 16 - 1);
+#pragma unroll
+        for (int i = 0; i < NL; i++)
+            v[i] = *(const mmq_i4 *)(s.q + (s.row[i] + c));
+        const int b = 8 * u + 2 * (ln & 3);
+        d0 = *(const uint16_t *)(s.d + 2u * (s.drow + min(b, nb - 1)));
+        d1 = *(const uint16_t *)(s.d + 2u * (s.drow + min(b + 1, nb - 1)));
+    }
+    __device__ __forceinline__ void store(uint8_t *l, int ln) const {
+#pragma unroll
+        for (int i = 0; i < NL; i++)
+            *(mmq_i4 *)(l + ((64 / CH) * i + ln / CH) * ROWB + 16 * (ln % CH)) = v[i];
+        *(uint32_t *)(l + 16 * ROWB + 4 * ln) = d0 | (d1 << 16);
+    }
+};
+
+template <int T> struct Mmw32Tile {
+    mmq_i4 q[4], d; // MFMA s: blocks 2s, 2s + 1; the row's eight f16 scales
+    __device__ __forceinline__ static Mmw32Tile read(const uint8_t *l, int r16, int q4) {
+        using B = Mmw32Blk<T>;
+        Mmw32Tile w;
+#pragma unroll
+        for (int s = 0; s < 4; s++)
+            w.q[s] = *(const mmq_i4 *)(l + r16 * B::ROWB + (B::Q8 ? 64 * s + 16 * q4 : 32 * s + 16 * (q4 >> 1)));
+        w.d = *(const mmq_i4 *)(l + 16 * B::ROWB + 16 * r16);
+        return w;
+    }
+};
+
+// One unit (nbu <= 8 blocks): acc[set][token pair] += its blocks' tails in order.
+// xs: the unit's scales, [MFMA s][token pair of both sets][token][block].
+template <int T>
+__device__ __forceinline__ void mmw32_acc(const Mmw32Tile<T> &w, int q4, int ns, int nbu, const mmq_i4 (&xa)[2][4],
+                                          const float4 *xs, float (&acc)[2][2]) {
+    const mmq_i4 z = {0, 0, 0, 0};
+#pragma unroll
+    for (int s = 0; s < 4; s++) {
+        if (2 * s >= nbu)
+            break;
+        mmq_i4 wv = w.q[s];
+        if constexpr (T == LH_Q4_0) { // the lane's nibble half, then q - 8 per byte: (q + 0x78) ^ 0x80
+            const uint32_t sh = 4 * (q4 & 1);
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+                wv[e] = (int)((((uint32_t)wv[e] >> sh) & 0x0F0F0F0Fu) + 0x78787878u) ^ (int)0x80808080u;
+        }
+        const float da = half_bits_to_float((uint32_t)w.d[s] & 0xffffu), db = half_bits_to_float((uint32_t)w.d[s] >> 16);
+        const bool two = 2 * s + 1 < nbu;
+#pragma unroll
+        for (int t = 0; t < 2; t++) {
+            if (t >= ns)
+                break;
+            const mmq_i4 dq = __builtin_amdgcn_mfma_i32_16x16x64_i8(xa[t][s], wv, z, 0, 0, 0);
+            const float4 xd = xs[8 * s + 4 * t + q4];
+            // d * xd * f32(dot)  (ggml.zig:1212-1218, 1289-1290)
+            const float a0 = da * xd.x, a1 = da * xd.z;
+            acc[t][0] = acc[t][0] + a0 * (float)dq[0];
+            acc[t][1] = acc[t][1] + a1 * (float)dq[2];
+            if (two) {
+                const float b0 = db * xd.y, b1 = db * xd.w;
+                acc[t][0] = acc[t][0] + b0 * (float)dq[1];
+                acc[t][1] = acc[t][1] + b1 * (float)dq[3];
+            }
+        }
+    }
+}
+
+// LDS: (XL: per work group; else per wave) the tokens' rows [16][xrow], 256
+// zeros, the scales [units][32] float4; per wave a unit of 16 weight rows.
+template <bool XL> __host__ __device__ constexpr int mmw32_xrow(int nb) { return (XL ? 32 * nb : 256) + 16; }
+template <bool XL> __host__ __device__ constexpr int mmw32_xbytes(int nb) {
+    return 16 * mmw32_xrow<XL>(nb) + 256 + (XL ? (nb + 7) / 8 : 1) * 512;
+}
+
+template <int T, bool FUSED, bool XL, int OCC>
+__global__ __launch_bounds__(64 * MMW_W, OCC) void mmw32_kernel(DmmvParams p) {
+    extern __shared__ __align__(16) uint8_t sh[];
+    using B = Mmw32Blk<T>;
+    constexpr int TOK = 16, M = FUSED ? 2 : 1, W = MMW_W;
+    const bool ident = p.ident_n > 0;
+    const int gi = blockIdx.y;
+    DmmvGroup grp;
+    if (ident) {
+        grp.plane = 0;
+        grp.first = gi * TOK;
+        grp.n = min(TOK, p.ident_n - grp.first);
+    } else {
+        const int ng = p.n_groups_dev ? *p.n_groups_dev : p.n_groups;
+        if (gi >= ng)
+            return;
+        grp = p.groups[gi];
+    }
+    const int n = grp.n, ns = (n + 7) / 8; // sets of 8 tokens
+    const int cols = p.cols, nb = cols / 32, nu = (nb + 7) / 8;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), ln = threadIdx.x & 63;
+    const int r16 = ln & 15, q4 = ln >> 4;
+    const int row0 = ((int)blockIdx.x * W + wave) * 16;
+    const int xrow = mmw32_xrow<XL>(nb), xbytes = mmw32_xbytes<XL>(nb);
+    uint8_t *wls = sh + (XL ? xbytes + wave * B::BYTES : wave * (xbytes + B::BYTES));
+    uint8_t *xl = XL ? sh : wls + B::BYTES;
+    uint8_t *zl = xl + TOK * xrow;
+    float *xds = (float *)(zl + 256);
+    // where token t's scale of block b goes: float4 (unit, MFMA, set, pair), element (token, block)
+    auto xd_at = [&](int t, int b) {
+        return (XL ? (b >> 3) * 128 : 0) + ((b >> 1) & 3) * 32 + (t >> 3) * 16 + ((t >> 1) & 3) * 4 + (t & 1) * 2 + (b & 1);
+    };
+    // the vector of the group's t-th token (past n: the last); group_src needs no group
+    const int *tab = p.group_src ? p.group_src + (size_t)gi * p.group_stride : p.pair_src + grp.first;
+    const int tmax = p.group_src ? TOK - 1 : n - 1;
+    auto vec_of = [&](int t) { return tab[min(t, tmax)]; };
+    typename B::Src src[M];
+    src[0] = B::src(p.w + (size_t)grp.plane * p.plane_bytes, p.rows, nb, row0, ln);
+    if constexpr (FUSED)
+        src[1] = B::src(p.w2 + (size_t)grp.plane * p.plane_bytes, p.rows, nb, row0, ln);
+    struct Stage {
+        B w[M];
+        mmq_i4 x[XL ? 1 : 4]; // (not XL) tokens 4 i + ln / 16, chunk ln % 16
+        float xd[2];          // tokens ln / 8, 8 + ln / 8, block ln % 8
+    } st[2];
+    const int8_t *xr[4];
+    const float *xdr[2];
+    if constexpr (!XL) {
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+            xr[i] = p.xq + (size_t)vec_of(4 * i + (ln >> 4)) * cols;
+#pragma unroll
+        for (int i = 0; i < 2; i++)
+            xdr[i] = p.xd + (size_t)vec_of(8 * i + (ln >> 3)) * nb;
+    }
+    auto load = [&](Stage &s, int u) {
+        s.w[0].load(src[0], u, nb, ln);
+        if constexpr (FUSED)
+            s.w[1].load(src[1], u, nb, ln);
+        if constexpr (!XL) {
+            const int c = 16 * min(16 * u + (ln & 15), 2 * nb - 1), b = min(8 * u + (ln & 7), nb - 1);
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+                s.x[i] = *(const mmq_i4 *)(xr[i] + c);
+#pragma unroll
+            for (int i = 0; i < 2; i++)
+                s.xd[i] = xdr[i][b];
+        }
+    };
+    auto commit = [&](const Stage &s, int m) { // matrix m's unit to this wave's LDS
+        wave_lds_sync();
+        s.w[m].store(wls, ln);
+        if constexpr (!XL)
+            if (m == 0) {
+#pragma unroll
+                for (int i = 0; i < 4; i++)
+                    *(mmq_i4 *)(xl + (4 * i + (ln >> 4)) * xrow + 16 * (ln & 15)) = s.x[i];
+#pragma unroll
+                for (int i = 0; i < 2; i++)
+                    xds[xd_at(8 * i + (ln >> 3), ln & 7)] = s.xd[i];
+            }
+        wave_lds_sync();
+    };
+    if constexpr (XL) {
+        // nb <= 64: four token rows per wave, all their loads before the weights' and the
+        // stores behind them, so one round trip covers the staging
+        int v[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+            v[i] = vec_of(4 * wave + i);
+        const int c0 = min(ln, 2 * nb - 1), c1 = min(64 + ln, 2 * nb - 1), cb = min(ln, nb - 1);
+        mmq_i4 x0[4], x1[4];
+        float xd[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            x0[i] = *(const mmq_i4 *)(p.xq + (size_t)v[i] * cols + 16 * c0);
+            x1[i] = *(const mmq_i4 *)(p.xq + (size_t)v[i] * cols + 16 * c1);
+            xd[i] = p.xd[(size_t)v[i] * nb + cb];
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        load(st[0], 0);
+        load(st[1], min(1, nu - 1));
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            uint8_t *l = xl + (size_t)(4 * wave + i) * xrow;
+            if (ln < 2 * nb)
+                *(mmq_i4 *)(l + 16 * ln) = x0[i];
+            if (64 + ln < 2 * nb)
+                *(mmq_i4 *)(l + 16 * (64 + ln)) = x1[i];
+            if (ln < nb)
+                xds[xd_at(4 * wave + i, ln)] = xd[i];
+        }
+        if (threadIdx.x < 16)
+            *(mmq_i4 *)(zl + 16 * threadIdx.x) = mmq_i4{0, 0, 0, 0};
+    } else {
+        load(st[0], 0);
+        load(st[1], min(1, nu - 1));
+        if (ln < 16)
+            *(mmq_i4 *)(zl + 16 * ln) = mmq_i4{0, 0, 0, 0};
+    }
+    lds_barrier();
+    // A row r16 = (token r16/2 of the set, block r16&1 of the span): live on the
+    // block's quarters, zeros elsewhere
+    const bool live = (q4 >> 1) == (r16 & 1);
+    const int xstep = XL && live ? 256 : 0;
+    const uint8_t *xt[2] = {live ? xl + (r16 / 2) * xrow + 16 * q4 : zl, live ? xl + (8 + r16 / 2) * xrow + 16 * q4 : zl};
+    float acc[M][2][2] = {};
+    // as mmw_kernel's step: the next tile is stored to LDS and read back under the arithmetic
+    commit(st[0], 0);
+    Mmw32Tile<T> w0 = Mmw32Tile<T>::read(wls, r16, q4);
+    auto step = [&](int u, Stage &cur, const Stage &nxt) {
+        const int nbu = min(8, nb - 8 * u);
+        mmq_i4 xa[2][4];
+#pragma unroll
+        for (int t = 0; t < 2; t++) {
+            if (t >= ns)
+                break;
+#pragma unroll
+            for (int s = 0; s < 4; s++) // (past the row's end: staged bytes of its clamped loads, or LDS never used)
+                xa[t][s] = *(const mmq_i4 *)(xt[t] + (2 * s < nbu ? u * xstep + 64 * s : 0));
+        }
+        Mmw32Tile<T> w1;
+        const float4 *xsp = (const float4 *)(xds + (XL ? u * 128 : 0));
+        if constexpr (FUSED) {
+            commit(cur, 1);
+            w1 = Mmw32Tile<T>::read(wls, r16, q4);
+            load(cur, min(u + 2, nu - 1)); // past the last unit: the last one again, not used
+            __builtin_amdgcn_sched_barrier(0);
+            mmw32_acc<T>(w0, q4, ns, nbu, xa, xsp, acc[0]);
+            if constexpr (XL) {
+                commit(nxt, 0);
+                w0 = Mmw32Tile<T>::read(wls, r16, q4);
+                mmw32_acc<T>(w1, q4, ns, nbu, xa, xsp, acc[M - 1]);
+            } else { // the unit's scales share the commit's LDS: after their last use
+                mmw32_acc<T>(w1, q4, ns, nbu, xa, xsp, acc[M - 1]);
+                commit(nxt, 0);
+                w0 = Mmw32Tile<T>::read(wls, r16, q4);
+            }
+        } else {
+            if constexpr (XL) {
+                commit(nxt, 0);
+                w1 = Mmw32Tile<T>::read(wls, r16, q4);
+                load(cur, min(u + 2, nu - 1));
+                __builtin_amdgcn_sched_barrier(0);
+                mmw32_acc<T>(w0, q4, ns, nbu, xa, xsp, acc[0]);
+                w0 = w1;
+            } else {
+                load(cur, min(u + 2, nu - 1));
+                __builtin_amdgcn_sched_barrier(0);
+                mmw32_acc<T>(w0, q4, ns, nbu, xa, xsp, acc[0]);
+                commit(nxt, 0);
+                w0 = Mmw32Tile<T>::read(wls, r16, q4);
+            }
+        }
+    };
+    for (int u = 0; u < nu; u += 2) {
+        step(u, st[0], st[1]);
+        if (u + 1 >= nu)
+            break;
+        step(u + 1, st[1], st[0]);
+    }
+    const int row = row0 + r16;
+    if (row >= p.rows)
+        return;
+#pragma unroll
+    for (int t = 0; t < 2; t++)
+#pragma unroll
+        for (int jj = 0; jj < 2; jj++) {
+            const int k = 8 * t + 2 * q4 + jj;
+            if (k >= n)
+                continue;
+            const float v = FUSED ? swiglu1(acc[0][t][jj], acc[M - 1][t][jj]) : acc[0][t][jj];
+            const int dst = ident || p.pos_ident ? grp.first + k : p.pair_dst[grp.first + k];
+            float *o = p.out + (size_t)dst * p.out_stride + row;
+            *o = p.accumulate ? *o + v : v;
+        }
+}
+
+template <int T, bool FUSED>
+static void mmw32_launch_t(const DmmvParams &p, hipStream_t st) {
+    const int groups = p.ident_n > 0 ? (p.ident_n + 15) / 16 : p.n_groups, nb = p.cols / 32;
+    const dim3 grid(((p.rows + 15) / 16 + MMW_W - 1) / MMW_W, groups), block(64 * MMW_W);
+    // waves per SIMD as registers (and for Q8_0 gate/up the LDS) allow
+    constexpr int OCC_XL = FUSED && T == LH_Q8_0 ? 2 : 3, OCC = FUSED ? 2 : 3;
+    if (p.cols <= MMW_XL_COLS)
+        hipLaunchKernelGGL((mmw32_kernel<T, FUSED, true, OCC_XL>), grid, block,
+                           (mmw32_xbytes<true>(nb) + MMW_W * Mmw32Blk<T>::BYTES), st, p);
+    else
+        hipLaunchKernelGGL((mmw32_kernel<T, FUSED, false, OCC>), grid, block,
+                           (MMW_W * (mmw32_xbytes<false>(nb) + Mmw32Blk<T>::BYTES)), st, p);
+}
+
+static bool is_k(int t) { return t == LH_Q4_K || t == LH_Q6_K; }
+
+// The one-shot kernels' shapes: K-quants in MmqOps registers and LDS sums,
+// 32-value blocks in mmq32_kernel's.
+static bool mmq_oneshot(int t, int cols, int max_tok, bool fused) {
+    if (!is_k(t))
         return mmq32_supported(t, cols, max_tok, fused);
-    if ((t != LH_Q4_K && t != LH_Q6_K) || cols % 256 || cols < 256 || max_tok < 1 || max_tok > 32)
+    if (cols % 256 || cols < 256 || max_tok < 1 || max_tok > 32)
         return false;
     if (fused && t != LH_Q4_K) // a fused pair is gate/up: Q4_K only here
         return false;
     int rg, ks, sbw;
     return mmq_shape(16, cols, (max_tok + 15) / 16, fused, rg, ks, sbw);
+}
+
+// The streamed kernels' shapes: whole blocks, byte offsets in 32 bits.
+static bool mmw_shape(int t, int rows, int cols, bool fused) {
+    if ((t != LH_Q4_K && t != LH_Q6_K && t != LH_Q8_0 && t != LH_Q4_0) || cols < block_elems(t) ||
+        cols % block_elems(t) || (fused && t == LH_Q6_K))
+        return false;
+    return (size_t)rows * (cols / block_elems(t)) * block_bytes(t) < ((size_t)1 << 32);
+}
+
+// (row tile, 16 lanes) pairs of a lane-group launch: the waves the streamed kernels run.
+static long lane_pairs(int rows, int n) { return (long)((rows + 15) / 16) * ((n + 15) / 16); }
+
+// Lane groups from MMW_MIN_WAVES pairs on (512 for a fused pair, twice the
+// bytes per wave) take the streamed kernel, below that the one-shot kernel
+// (8 waves to a row tile) where it serves the shape: too few waves stream.
+// Measured, us per launch, one-shot / streamed: Q4_K 8192 x 4096 at 16 lanes
+// (512 pairs) 14.4 / 15.1, at 32 (1024) 22.6 / 15.8; 7168 x 2048 at 24 (896)
+// 13.1 / 9.8; Q6_K 16384 x 4096 at 16 (1024) 32.7 / 20.6; fused 2048 x 7168 at
+// 24 (256) 25.6 / 32.1, at 64 (512) 44.8 / 32.6; fused 4096 x 2048 at 24 (512)
+// 12.7 / 13.2, at 64 (1024) 20.4 / 14.0.
+constexpr long MMW_MIN_WAVES = 768, MMW_MIN_WAVES_FUSED = 512;
+static bool lanes_streamed(int t, int rows, int cols, int n, bool fused) {
+    return mmw_shape(t, rows, cols, fused) &&
+           lane_pairs(rows, n) >= (fused ? MMW_MIN_WAVES_FUSED : MMW_MIN_WAVES);
+}
+
+// n vectors against one [rows][cols] matrix (or a fused pair): whether the
+// matrix cores take them from the dot4 matvec.  By type and size, us per
+// launch, dot4 / matrix cores: Q4_K 4096 x 4096 at 5 vectors 11.4 / 9.1,
+// 1024 x 2048 6.7 / 6.6; Q6_K at 5 10.8 / 10.4 and 6.6 / 7.1, at 8 12.5 /
+// 10.6 and 7.8 / 7.2; Q8_0 at 5 15.2 / 10.0 and 7.8 / 8.5, at 8 19.7 / 10.5
+// and 9.8 / 8.8 (Q4_0 8.9 / 8.7); 768 x 288 at 32 6.2 / 7.4.  A shape only the
+// streamed kernels serve needs their rows staged whole or 512 pairs (Q8_0
+// 4096 x 11008 at 16 vectors, 256 pairs, 60.5 / 56.5, Q4_0 47.9 / 58.2; at
+// 32, 512 pairs, 111 / 57 and 84 / 59).  A fused pair: from 16 as measured
+// for Q4_K (2048 x 7168 at 8 vectors 16 / 24, at 24 47 / 25).
+bool mmq_dense(int t, int rows, int cols, int n, bool fused) {
+    if (rows < 1 || n < 1)
+        return false;
+    const int min_k = fused ? 16 : t == LH_Q4_K ? 5 : 8;
+    const size_t size = (size_t)rows * cols;
+    const int min_32 = size >= ((size_t)8 << 20) ? 5 : size >= ((size_t)1 << 20) ? 8 : 64;
+    if (n < (is_k(t) ? min_k : min_32))
+        return false;
+    if (mmq_oneshot(t, cols, 16, fused))
+        return true;
+    return mmw_shape(t, rows, cols, fused) &&
+           (lane_pairs(rows, n) >= 512 || (!is_k(t) && !fused && cols <= MMW_XL_COLS));
+}
+
+// The expert matmuls of n tokens: whether they run on the matrix cores in
+// groups of 16.  By type and expert size, us per layer with the dot4 / matrix
+// core matmuls, Zipf-skewed router: Q4_K + Q6_K 2048 x 768 x 128 at 5 tokens
+// 48.8 / 46.4 (uniform 58.3 / 56.8), 1024 x 512 x 32 at 8 32.4 / 32.9, at 10
+// 35.2 / 34.0; Q8_0 2048 x 768 at 8 66.7 / 61.7 (uniform 79.3 / 86.7), at 12
+// 90.5 / 66.2 (113 / 97), Q4_0 at 12 76.3 / 57.5; 7168 x 2048 x 16 at 5 Q8_0
+// 183 / 150, Q4_0 142 / 116; Q8_0 1024 x 512 x 32 at 15 35.2 / 40.1.
+static int experts_min(int t, size_t size) {
+    if (is_k(t))
+        return size >= 1500000 ? 5 : 10;
+    return size >= 8000000 ? 5 : size >= 1500000 ? 12 : 20;
+}
+bool mmq_experts(int gate_t, int down_t, int dim, int ffn, int n) {
+    const size_t size = (size_t)dim * ffn;
+    return mmw_shape(gate_t, ffn, dim, true) && mmw_shape(down_t, dim, ffn, false) && n >= experts_min(gate_t, size) &&
+           n >= experts_min(down_t, size);
 }
 
 template <int T, int MT, bool FUSED>
@@ -1198,7 +1579,7 @@ bool launch_mmq_seg(DmmvSegParams sp, hipStream_t st) {
     constexpr int mt = 1;
     int rg = MMQ_WAVES, ks = 0, sbw = 0, tiles = 0;
     for (int i = 0; i < sp.n_seg; i++) {
-        if ((sp.seg[i].t != LH_Q4_K && sp.seg[i].t != LH_Q6_K) || !mmq_supported(sp.seg[i].t, p.cols, 16 * mt, false))
+        if (!is_k(sp.seg[i].t) || !mmq_oneshot(sp.seg[i].t, p.cols, 16 * mt, false))
             return false;
         int r, k, b;
         if (!mmq_shape(sp.seg[i].rows, p.cols, mt, false, r, k, b))
@@ -1223,17 +1604,30 @@ bool launch_mmq_seg(DmmvSegParams sp, hipStream_t st) {
 }
 
 // Groups of at most max_tok (<= 32) tokens (with p.ident_n: max_tok sets
-// the group size); p.rpw is unused.
+// the group size); p.rpw is unused.  Expert groups (<= 16 tokens) stream.
 bool launch_mmq(int t, int max_tok, bool fused, const DmmvParams &p, hipStream_t st) {
-    if (!mmq_supported(t, p.cols, max_tok, fused) || p.rows < 1)
+    if (p.rows < 1 || max_tok < 1 || max_tok > 32)
         return false;
-    if (t == LH_Q8_0 || t == LH_Q4_0) {
-        launch_mmq32(t, max_tok, p, st);
+    if (p.ident_n > 0 && max_tok > 16 && !mmq_oneshot(t, p.cols, max_tok, fused))
+        max_tok = 16; // the one-shot kernel's registers hold 16 tokens of the widest rows
+    const bool oneshot = mmq_oneshot(t, p.cols, max_tok, fused);
+    const bool stream = p.ident_n > 0 ? lanes_streamed(t, p.rows, p.cols, p.ident_n, fused) ||
+                                            (!oneshot && mmw_shape(t, p.rows, p.cols, fused))
+                                      : max_tok <= 16 && mmw_shape(t, p.rows, p.cols, fused);
+    if (!stream && !oneshot)
+        return false;
+    const int mt = max_tok > 16 ? 2 : 1;
+    if (!is_k(t)) {
+        if (!stream)
+            launch_mmq32(t, max_tok, p, st);
+        else if (t == LH_Q8_0)
+            fused ? mmw32_launch_t<LH_Q8_0, true>(p, st) : mmw32_launch_t<LH_Q8_0, false>(p, st);
+        else
+            fused ? mmw32_launch_t<LH_Q4_0, true>(p, st) : mmw32_launch_t<LH_Q4_0, false>(p, st);
         note_launch();
         return true;
     }
-    const int mt = max_tok > 16 ? 2 : 1;
-    if (mmw_serves(t, fused, p)) {
+    if (stream) {
         if (t == LH_Q4_K)
             fused ? mmw_launch_t<LH_Q4_K, 1, true>(p, st) : mmw_launch_t<LH_Q4_K, 1, false>(p, st);
         else if (mt == 1)

@@ -116,9 +116,9 @@ int dense_ffn_add(const DenseFfn &f, const float *x, size_t n, size_t dim, float
     p.n_groups = ng;
     p.out = act;
     p.out_stride = (int)f.ffn;
-    // from MMQ_MIN_TOK tokens each matmul runs on the matrix cores where its type and shape are
-    // served (7168 -> 2048 -> 7168 Q4_K at 24 tokens: gate/up 48 -> 25 us, down 33 -> 10 us)
-    const bool mq = use_mmq(f.gate_t, (int)dim, (int)n, 16, true);
+    // each matmul on the matrix cores where mmq_dense takes it
+    // (7168 -> 2048 -> 7168 Q4_K at 24 tokens: gate/up 48 -> 25 us, down 33 -> 10 us)
+    const bool mq = mmq_dense(f.gate_t, (int)f.ffn, (int)dim, (int)n, true);
     p.ident_n = mq ? (int)n : 0;
     p.rpw = mq ? 0 : dmmv_pick_rpw(f.gate_t, (int)dim, (int)f.ffn, ng, nt, true);
     if (!(mq ? launch_mmq(f.gate_t, 16, true, p, st) : launch_dmmv(f.gate_t, nt, true, p, st)))
@@ -138,10 +138,10 @@ int dense_ffn_add(const DenseFfn &f, const float *x, size_t n, size_t dim, float
     d.out = out;
     d.out_stride = (int)dim;
     d.accumulate = add ? 1 : 0; // add: out = out + value
-    const bool mqd = use_mmq(f.down_t, (int)f.ffn, (int)n, 32, false);
+    const bool mqd = mmq_dense(f.down_t, (int)dim, (int)f.ffn, (int)n, false);
     d.ident_n = mqd ? (int)n : 0;
     d.rpw = mqd ? 0 : dmmv_pick_rpw(f.down_t, (int)f.ffn, (int)dim, ng, nt, false);
-    if (!(mqd ? launch_mmq(f.down_t, 32, false, d, st) : launch_dmmv(f.down_t, nt, false, d, st)))
+    if (!(mqd ? launch_mmq(f.down_t, n > 16 ? 32 : 16, false, d, st) : launch_dmmv(f.down_t, nt, false, d, st)))
         return fail(LOOMHIP_ERR_ARG, "shared expert: down partials exceed LDS");
     return LOOMHIP_OK;
 }
@@ -205,10 +205,9 @@ static int moe_run(const MoeRun &m, const float *normed, const float *logits_in,
                     "on a normalised input");
     const size_t P = n * m.k;
     const bool decode = n <= DECODE_MAX_TOK && decode_supported(m.gate_t, m.down_t, (int)m.ffn);
-    // matrix cores for the expert matmuls from MMQ_MIN_TOK tokens on, groups
+    // matrix cores for the expert matmuls where mmq_experts takes them, groups
     // of up to 16 tokens per expert
-    const bool mq = !decode && use_mmq(m.gate_t, (int)m.dim, (int)n, 16, true) &&
-                    use_mmq(m.down_t, (int)m.ffn, (int)n, 16, false);
+    const bool mq = !decode && mmq_experts(m.gate_t, m.down_t, (int)m.dim, (int)m.ffn, (int)n);
     const int nt = mq ? 16 : moe_nt(n, m.k, m.E);
     const int maxg = moe_max_groups((int)n, (int)m.k, (int)m.E, nt);
     // workspace layout
@@ -223,10 +222,12 @@ static int moe_run(const MoeRun &m, const float *normed, const float *logits_in,
     const size_t o_ids = take(P * 4), o_gates = take(P * 4);
     const size_t o_ptok = take(P * 4), o_pof = take(P * 4), o_iota = take(P * 4);
     const size_t o_groups = take(maxg * sizeof(DmmvGroup)), o_ng = take(16);
-    const size_t o_gsrc = take(mq ? (size_t)maxg * nt * 4 : 0);
     const size_t o_act = take(P * m.ffn * 4);
     const size_t o_qa = take(qbytes(P, m.ffn));
     const size_t o_y = take(decode ? 0 : P * m.dim * 4);
+    // the groups' token rows: an aid, left out where a fixed workspace has no room for them
+    const bool gsrc = mq && !(ws && off + align16((size_t)maxg * nt * 4) > ws_cap);
+    const size_t o_gsrc = take(gsrc ? (size_t)maxg * nt * 4 : 0);
     char *base;
     if (ws) {
         if (off > ws_cap)
@@ -322,7 +323,7 @@ static int moe_run(const MoeRun &m, const float *normed, const float *logits_in,
     b.iota = (int *)(base + o_iota);
     b.groups = (DmmvGroup *)(base + o_groups);
     b.n_groups = (int *)(base + o_ng);
-    b.group_src = mq ? (int *)(base + o_gsrc) : nullptr;
+    b.group_src = gsrc ? (int *)(base + o_gsrc) : nullptr;
     float *y = (float *)(base + o_y);
     gp.b = b;
     gp.chain = 1;

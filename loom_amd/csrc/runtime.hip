@@ -225,8 +225,8 @@ int matvec_dev_impl(int t, float *out, const void *w, const float *x, size_t n, 
     qa.d = (float *)((char *)g_ctx.act.ptr + align16(n * cols));
     qa.s = (int32_t *)((char *)qa.d + align16(n * cols / 32 * 4));
     launch_quant_act(t, x, (int)cols, (int)cols, (int)n, qa, st);
-    const bool mq = use_mmq(t, (int)cols, (int)n, 32, false);
-    const int nt = mq ? 32 : pick_nt((int)n);
+    const bool mq = mmq_dense(t, (int)rows, (int)cols, (int)n, false);
+    const int nt = mq ? (n > 16 ? 32 : 16) : pick_nt((int)n);
     int ng = 0;
     const DmmvGroup *groups = dense_groups((int)n, nt, &ng);
     if (!groups)

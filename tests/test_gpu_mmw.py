@@ -87,3 +87,53 @@ def test_dense_ffn_frame_on_matrix_cores(oracle, n):
     dm = lh.DeviceModel.synth(spec, seed=17, keep_ggml=True)
     rels, same = _batch_steps(lh, OracleModel(oracle, dm), dm, n, 2, 60, seed=n)
     assert rels.max() == 0.0 and same
+
+
+Q4_0, Q8_0 = 2, 8
+
+
+# lane groups of 32-value blocks that stream: at least 768 (row tile, 16 vectors)
+# pairs, or a shape the one-shot kernel does not hold
+@pytest.mark.parametrize("t", [Q4_0, Q8_0])
+@pytest.mark.parametrize("rows,cols,n", [(8192 + 5, 288, 16), (8192 + 17, 2080, 20), (12288 + 1, 2048, 9),
+                                         (12288 + 15, 4096, 16), (16384, 32, 65), (8192 + 33, 4384, 33),
+                                         (1100, 1952, 8)])
+def test_streamed_32_block_matmul_edges(be, oracle, t, rows, cols, n):
+    """Odd block counts (9, 65, 137, 61), units of fewer than 8 blocks, one
+    block per row, partial token sets and groups, rows staged whole and not."""
+    rng = np.random.default_rng(rows + cols + n + t)
+    raw = npref.pinned_scale_blocks(t, rows, cols, rng)
+    xs = np.stack([oracle.normal(cols, 100 * n + k, 0.0, float(k % 5 + 1)) for k in range(n)])
+    _check(be, oracle, t, raw, xs, rows, cols)
+
+
+# five to fifteen vectors on the matrix cores (one-shot), rows too wide for 32 lanes a wave
+@pytest.mark.parametrize("t,rows,cols,n", [(Q4_K, 300, 2048, 5), (Q4_K, 77, 8192, 17), (Q6_K, 300, 768, 8),
+                                           (Q6_K, 130, 8192, 9), (Q8_0, 2100, 4096, 5), (Q4_0, 1100, 1024, 11),
+                                           (Q4_K, 4100, 11008, 32), (Q6_K, 8200, 8448, 16)])
+def test_matmul_from_five_vectors(be, oracle, t, rows, cols, n):
+    rng = np.random.default_rng(rows + cols + n + t)
+    raw = npref.pinned_scale_blocks(t, rows, cols, rng)
+    xs = np.stack([oracle.normal(cols, 100 * n + k, 0.0, float(k % 5 + 1)) for k in range(n)])
+    _check(be, oracle, t, raw, xs, rows, cols)
+
+
+@pytest.mark.parametrize("t,dim,ffn,n", [(Q8_0, 288, 96, 21), (Q4_0, 544, 288, 40), (Q8_0, 2080, 768, 12),
+                                         (Q4_0, 1024, 1536, 13), (Q4_K, 512, 256, 10), (Q4_K, 2304, 768, 5)])
+def test_moe_layer_streamed_experts(be, oracle, t, dim, ffn, n):
+    """The routed layer with its expert matmuls streamed in groups of 16 for
+    every type: ids, gates and output bits against lo_moe_batch_union."""
+    import torch
+    from test_gpu_moe import _dev_layer, make_layer
+
+    E, k = 6, 3
+    w = make_layer(oracle, dim, ffn, E, k, seed=dim + n, gate_t=t, down_t=t)
+    layer = _dev_layer(be, w)
+    xs = np.stack([oracle.normal(dim, 700 + i, 0.0, 1.0) for i in range(n)])
+    resid = np.stack([oracle.normal(dim, 900 + i, 0.0, 1.0) for i in range(n)])
+    out, ids = torch.from_numpy(resid.copy()).cuda(), torch.empty((n, k), dtype=torch.int32, device="cuda")
+    layer(torch.from_numpy(xs).cuda(), out, combine=be.COMBINE_EXPERT_ASC, ids=ids)
+    want, wid, _ = oracle.moe_batch_union(w, xs, resid)
+    torch.cuda.synchronize()
+    assert np.array_equal(ids.cpu().numpy().astype(np.uint32), wid)
+    assert np.array_equal(out.cpu().numpy().view(np.uint32), want.view(np.uint32))
