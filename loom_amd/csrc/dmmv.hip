@@ -25,7 +25,7 @@ namespace lh {
 // FUSED), written to lds[((m * NT + k) * TR + rl) * nb + b] for matrix m.
 // The activations may live in global memory or in LDS (generic pointers).
 template <int T, int NT, bool FUSED>
-__device__ inline void tile_partials(const uint8_t *wb, const uint8_t *wb2, int rows, int cols,
+__device__ __forceinline__ void tile_partials(const uint8_t *wb, const uint8_t *wb2, int rows, int cols,
                                      const int8_t *xq, const float *xd, const int32_t *xs,
                                      const int *vec, int n, int row0, int rpw, float *lds) {
     using F = Fmt<T>;
@@ -126,7 +126,9 @@ __device__ inline void tile_partials(const uint8_t *wb, const uint8_t *wb2, int 
 
 // ---- grouped matvec: one work group per (row tile, group of <= NT vectors
 // sharing one weight plane) -------------------------------------------------------
-template <int T, int NT, bool FUSED>
+// SLOTS: the group's vectors are slots 0 .. n - 1 of p's activations (a
+// work group's own), else pair_src says which.
+template <int T, int NT, bool FUSED, bool SLOTS = false>
 __device__ __forceinline__ void dmmv_tile(const DmmvParams &p, int tile, int group, float *lds, int *vec) {
     using F = Fmt<T>;
     const DmmvGroup g = p.groups[group];
@@ -134,8 +136,10 @@ __device__ __forceinline__ void dmmv_tile(const DmmvParams &p, int tile, int gro
     const int nb = p.cols / F::BE;
     const int TR = WAVES * p.rpw;
     const int row0 = tile * TR;
-    if (threadIdx.x < NT)
-        vec[threadIdx.x] = p.pair_src[g.first + ((int)threadIdx.x < n ? threadIdx.x : 0)];
+    if (threadIdx.x < NT) {
+        const int k = (int)threadIdx.x < n ? threadIdx.x : 0;
+        vec[threadIdx.x] = SLOTS ? k : p.pair_src[g.first + k];
+    }
     __syncthreads();
     const uint8_t *wb = p.w + (size_t)g.plane * p.plane_bytes;
     const uint8_t *wb2 = FUSED ? p.w2 + (size_t)g.plane * p.plane_bytes : nullptr;
@@ -197,34 +201,50 @@ __global__ __launch_bounds__(256) void dmmv_seg_kernel(DmmvSegParams sp) {
     }
 }
 
-// ---- the attention rmsnorm fused into q, k and v (PARITY, one vector) -----------
-// Every work group normalises x itself (the reference's sequential sum of the
-// squares, 4 waves) and quantizes the row for the segments' activation block
-// into LDS, then runs dmmv_seg_kernel's tile against that LDS copy: the norm
-// launch, its HBM round trip of the int8 row and one launch gap leave the
-// layer.  Same values as norm_quant_kernel<QB, true> followed by
-// dmmv_seg_kernel<1>.
+// ---- one vector per group: its int8 form made by the matvec's own work groups -----
+// A matvec of one vector is a chain of short launches, quant_act's 2.3 us and
+// dmmv's 4.5 at 768 x 2048.  Here every work group quantizes its group's
+// vector into LDS and runs the tile against it: one launch, and no round trip
+// of the int8 row.  NORM: x is first normalised by the reference's rmsnorm
+// (the sequential sum of the squares, 4 waves), every work group for itself --
+// the attention norm with q, k and v, the FFN norm with gate and up.  The
+// stories15M token (6 layers, dim 288): 66 -> 42 launches, 292 -> 230 us; a
+// matvec call from Python 10.8 -> 7.4 us at 768 x 2048.  Same values as norm_quant_kernel / quant_act_kernel followed by dmmv_seg_kernel
+// or dmmv_kernel.
 constexpr int NSEG_MAX_DIM = 4096;
 constexpr int NSEG_XV = norm_xv(NSEG_MAX_DIM, 4);
 
-__global__ __launch_bounds__(256) void norm_seg_kernel(DmmvSegParams sp, const float *__restrict__ x,
-                                                       const float *__restrict__ nw, float eps) {
-    extern __shared__ float lds[];
+// LDS bytes of a quantized vector.
+static __host__ __device__ size_t self_act_bytes(int cols) {
+    return align16((size_t)cols) + align16((size_t)(cols / 32) * 4) + (size_t)(cols / 16) * 4;
+}
+
+template <bool FUSED, bool NORM>
+__global__ __launch_bounds__(256, 4) void dmmv_self_kernel(DmmvSegParams sp, const float *__restrict__ x, int x_stride,
+                                                        const float *__restrict__ nw, float eps, int lds_part) {
+    extern __shared__ __align__(16) float lds[];
     __shared__ int vec[1];
-    __shared__ __align__(16) float xn[NSEG_MAX_DIM];
-    __shared__ SeqSumLds seq;
-    __shared__ __align__(16) int8_t aq[NSEG_MAX_DIM];
-    __shared__ float ad[NSEG_MAX_DIM / 32];
-    __shared__ int32_t as[NSEG_MAX_DIM / 16];
-    const int dim = sp.base.cols;
-    float4 xv[NSEG_XV], wv[NSEG_XV];
-    norm_exact_load<4, NSEG_XV>(x, nw, dim, xv, wv);
-    norm_exact_block<4, NSEG_XV>(xv, wv, dim, eps, xn, seq);
-    // the row for the segments' weight type (they share its activation block)
-    const int qt = sp.seg[0].t;
-    const int items = quant_items(qt, dim);
-    for (int it = (int)threadIdx.x >> 6; it < items; it += 4)
-        quant_item_wave(qt, xn, dim, 0, it, QAct{aq, ad, as});
+    const int cols = sp.base.cols, wave = (int)threadIdx.x >> 6;
+    int8_t *aq = (int8_t *)lds + lds_part;
+    QAct qa;
+    qa.q = aq;
+    qa.d = (float *)(aq + align16((size_t)cols));
+    qa.s = (int32_t *)((char *)qa.d + align16((size_t)(cols / 32) * 4));
+    const int qt = sp.seg[0].t; // the segments share its activation block
+    const int items = quant_items(qt, cols);
+    if constexpr (NORM) {
+        __shared__ __align__(16) float xn[NSEG_MAX_DIM];
+        __shared__ SeqSumLds seq;
+        float4 xv[NSEG_XV], wv[NSEG_XV];
+        norm_exact_load<4, NSEG_XV>(x, nw, cols, xv, wv);
+        norm_exact_block<4, NSEG_XV>(xv, wv, cols, eps, xn, seq);
+        for (int it = wave; it < items; it += 4)
+            quant_item_wave(qt, xn, cols, 0, it, qa);
+    } else {
+        const float *xv = x + (size_t)sp.base.pair_src[sp.base.groups[blockIdx.y].first] * x_stride;
+        for (int it = wave; it < items; it += 4)
+            quant_item_wave(qt, xv, cols, 0, it, qa);
+    }
     lds_barrier();
     int s = 0, bx = blockIdx.x;
     while (s + 1 < sp.n_seg && bx >= sp.seg[s].tiles) {
@@ -237,46 +257,61 @@ __global__ __launch_bounds__(256) void norm_seg_kernel(DmmvSegParams sp, const f
     p.rpw = sp.seg[s].rpw;
     p.out = sp.seg[s].out;
     p.out_stride = sp.seg[s].rows;
-    p.xq = aq;
-    p.xd = ad;
-    p.xs = as;
+    p.xq = qa.q;
+    p.xd = qa.d;
+    p.xs = qa.s;
     switch (sp.seg[s].t) {
     case LH_Q4_K:
-        dmmv_tile<LH_Q4_K, 1, false>(p, bx, 0, lds, vec);
+        dmmv_tile<LH_Q4_K, 1, FUSED, true>(p, bx, blockIdx.y, lds, vec);
         break;
     case LH_Q6_K:
-        dmmv_tile<LH_Q6_K, 1, false>(p, bx, 0, lds, vec);
+        dmmv_tile<LH_Q6_K, 1, FUSED, true>(p, bx, blockIdx.y, lds, vec);
         break;
     case LH_Q8_0:
-        dmmv_tile<LH_Q8_0, 1, false>(p, bx, 0, lds, vec);
+        dmmv_tile<LH_Q8_0, 1, FUSED, true>(p, bx, blockIdx.y, lds, vec);
         break;
     default:
-        dmmv_tile<LH_Q4_0, 1, false>(p, bx, 0, lds, vec);
+        dmmv_tile<LH_Q4_0, 1, FUSED, true>(p, bx, blockIdx.y, lds, vec);
         break;
     }
 }
 
-// One vector (sp.base: n_groups 1, identity pairs): false = not served (the
-// caller normalises and runs launch_dmmv_seg instead).
-bool launch_norm_seg(DmmvSegParams sp, const float *x, const float *norm_w, float eps, hipStream_t st) {
-    const int dim = sp.base.cols;
-    if (dim > NSEG_MAX_DIM || dim % 256 || sp.base.n_groups != 1 || sp.n_seg < 1)
+// Up to DMMV_MAX_SEG matrices (or one fused pair, base.w2) against groups of
+// one of the vectors x; norm_w: one group, normalised first.  False = not
+// served (nothing launched; the caller quantizes apart): LDS, rows so long or
+// work groups so many that each one's repeated quantization (or norm) costs
+// more than the launch it saves.  Measured, us back to back, two launches /
+// one: 768 x 2048 and 2048 x 2048 Q4_0 5.95 / 5.50 and 6.03 / 5.57, Q4_K 5.51
+// / 5.14 and 5.50 / 5.18; 8192 x 2048 (1024 work groups) Q4_K 6.36 / 7.12;
+// 4096 x 4096 6.61 / 7.72; two vectors per group 768 x 2048 6.03 / 6.51.
+constexpr int SELF_MAX_COLS = 2048, SELF_MAX_WGS = 512, SELF_MAX_WGS_NORM = 640;
+bool launch_dmmv_self(bool fused, DmmvSegParams sp, const float *x, int x_stride, const float *norm_w, float eps,
+                      hipStream_t st) {
+    const int cols = sp.base.cols;
+    if (sp.n_seg < 1 || (fused && sp.n_seg != 1) || sp.base.n_groups_dev ||
+        (norm_w ? sp.base.n_groups != 1 || cols > NSEG_MAX_DIM || cols % 32 : cols > SELF_MAX_COLS))
         return false;
-    size_t lds = 0;
+    size_t part = 0;
     int tiles = 0;
     for (int i = 0; i < sp.n_seg; i++) {
         DmmvSeg &g = sp.seg[i];
-        if (act_block(g.t) != act_block(sp.seg[0].t))
+        if (act_block(g.t) != act_block(sp.seg[0].t) || !dmmv_supported(g.t, cols))
             return false;
-        g.rpw = dmmv_pick_rpw(g.t, dim, g.rows, 1, 1, false);
+        g.rpw = dmmv_pick_rpw(g.t, cols, g.rows, sp.base.n_groups, 1, fused);
         g.tiles = (g.rows + WAVES * g.rpw - 1) / (WAVES * g.rpw);
         tiles += g.tiles;
-        const size_t l = dmmv_lds_bytes(g.t, dim, 1, false, g.rpw);
-        lds = l > lds ? l : lds;
+        const size_t l = dmmv_lds_bytes(g.t, cols, 1, fused, g.rpw);
+        part = l > part ? l : part;
     }
-    if (lds > 64 * 1024)
+    part = align16(part);
+    const size_t lds = part + self_act_bytes(cols);
+    const long wgs = (long)tiles * sp.base.n_groups, max_wgs = norm_w ? SELF_MAX_WGS_NORM : SELF_MAX_WGS;
+    if (lds > 64 * 1024 || ((!norm_w || fused) && wgs > max_wgs)) // (the q/k/v launch: at any size)
         return false;
-    hipLaunchKernelGGL(norm_seg_kernel, dim3(tiles), dim3(256), lds, st, sp, x, norm_w, eps);
+    const dim3 grid(tiles, sp.base.n_groups);
+    auto kern = norm_w ? (fused ? dmmv_self_kernel<true, true> : dmmv_self_kernel<false, true>)
+                       : (fused ? dmmv_self_kernel<true, false> : dmmv_self_kernel<false, false>);
+    hipLaunchKernelGGL(kern, grid, dim3(256), lds, st, sp, x, x_stride, norm_w, eps, (int)part);
     note_launch();
     return true;
 }

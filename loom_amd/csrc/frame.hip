@@ -1144,6 +1144,27 @@ static bool frame_matvec(int t, const void *wt, int rows, int cols, const FrameW
     return ok;
 }
 
+// A matvec (w2: a fused pair) of one lane's f32 row x, quantized -- with norm_w
+// normalised first -- by the launch itself; false = not served.
+static bool frame_self(int t, const void *wt, const void *w2, int rows, int cols, const FrameWs &w,
+                       const float *x, const float *norm_w, float eps, float *out, int accumulate, hipStream_t st,
+                       int tag) {
+    DmmvSegParams sp{};
+    sp.base.w2 = (const uint8_t *)w2;
+    sp.base.cols = cols;
+    sp.base.pair_src = g_ctx.iota;
+    sp.base.pair_dst = g_ctx.iota;
+    sp.base.groups = w.groups;
+    sp.base.n_groups = w.n_groups;
+    sp.base.accumulate = accumulate;
+    sp.seg[0] = DmmvSeg{(const uint8_t *)wt, t, rows, out, 0, 0};
+    sp.n_seg = 1;
+    const int ph = prof_begin(tag, st);
+    const bool ok = launch_dmmv_self(w2 != nullptr, sp, x, cols, norm_w, eps, st);
+    prof_end(ph, st);
+    return ok;
+}
+
 // us per two-layer step (Qwen3-30B-A3B shapes), dot4 / matrix-core q, k, v: 5 lanes 336.6 / 332.9,
 // 15 lanes 349.5 / 332.7
 constexpr size_t QKV_MMQ_MIN = 5;
@@ -1173,7 +1194,7 @@ static bool frame_qkv(const loomhip_layer &l, const FrameDims &D, const FrameWs 
         if (n != 1)
             return false;
         const int ph = prof_begin(LOOMHIP_KT_QKV, st);
-        *fused = launch_norm_seg(sp, w.x, l.attn_norm, D.eps, st);
+        *fused = launch_dmmv_self(false, sp, w.x, 0, l.attn_norm, D.eps, st);
         prof_end(ph, st);
         return *fused;
     }
@@ -1365,6 +1386,7 @@ int frame_layer(const FrameCall &c, const loomhip_layer &l, size_t li, uint32_t 
         note_launch();
     }
     const float *qin = fuse_rope ? w.q : w.qrot;
+    bool wo_self = false; // wo's launch quantizes its input itself
     if (parity) {
         // the reference's own order over the whole context: scores, softmax, P.V
         // few lanes: P.V quantizes wo's input itself
@@ -1372,7 +1394,8 @@ int frame_layer(const FrameCall &c, const loomhip_layer &l, size_t li, uint32_t 
         if (!launch_attn_exact(D, qin, w.k, w.v, l.q_norm, l.k_norm, c.rope_cs, c.kc, c.vc, c.pos, (int)li,
                                fuse_rope, w.S, w.s_stride, w.att, n, qfuse ? l.wo_t : -1, w.qa_att, st))
             return fail(LOOMHIP_ERR_ARG, "token_frame: exact attention declined");
-        if (!qfuse)
+        wo_self = !qfuse && n == 1;
+        if (!qfuse && !wo_self)
             launch_quant_act(l.wo_t, w.att, D.qd, D.qd, (int)n, w.qa_att, st);
     } else {
         const int ph = prof_begin(LOOMHIP_KT_ATTN, st);
@@ -1410,7 +1433,11 @@ int frame_layer(const FrameCall &c, const loomhip_layer &l, size_t li, uint32_t 
                                D, w.part, c.pos, n_rec, span, direct ? 1 : 0, w.qa_att);
         note_launch();
     }
-    if (!frame_matvec(l.wo_t, l.wo, D.dim, D.qd, w, n, w.qa_att, w.x, 1, st, LOOMHIP_KT_WO, true, 16))
+    if (wo_self && !frame_self(l.wo_t, l.wo, nullptr, D.dim, D.qd, w, w.att, nullptr, 0.0f, w.x, 1, st, LOOMHIP_KT_WO)) {
+        launch_quant_act(l.wo_t, w.att, D.qd, D.qd, (int)n, w.qa_att, st);
+        wo_self = false;
+    }
+    if (!wo_self && !frame_matvec(l.wo_t, l.wo, D.dim, D.qd, w, n, w.qa_att, w.x, 1, st, LOOMHIP_KT_WO, true, 16))
         return fail(LOOMHIP_ERR_ARG, "token_frame: wo matvec declined");
     // FFN block (llama.zig:1203-1224)
     if (l.is_moe) {
@@ -1423,7 +1450,12 @@ int frame_layer(const FrameCall &c, const loomhip_layer &l, size_t li, uint32_t 
         // the batched combine also forms the next rmsnorm of x (next)
         return moe_layer_next_norm(&l.moe, w.normed, n, combine, w.x, ids, next, next_done, st);
     }
-    launch_norm(act_block(l.ffn_gate_t), w.x, D.dim, l.ffn_norm, D.eps, w.qa_dim, nullptr, n, st, parity);
+    // one lane in PARITY: the gate/up launch normalises its input itself
+    const bool gu_self = parity && n == 1 &&
+                         frame_self(l.ffn_gate_t, l.ffn_gate, l.ffn_up, (int)l.ffn, D.dim, w, w.x, l.ffn_norm, D.eps,
+                                    w.act, 0, st, -1);
+    if (!gu_self)
+        launch_norm(act_block(l.ffn_gate_t), w.x, D.dim, l.ffn_norm, D.eps, w.qa_dim, nullptr, n, st, parity);
     DmmvParams p{};
     p.w = (const uint8_t *)l.ffn_gate;
     p.w2 = (const uint8_t *)l.ffn_up;
@@ -1441,8 +1473,11 @@ int frame_layer(const FrameCall &c, const loomhip_layer &l, size_t li, uint32_t 
     const bool mq = mmq_dense(l.ffn_gate_t, (int)l.ffn, D.dim, (int)n, true);
     p.ident_n = mq ? (int)n : 0;
     p.rpw = mq ? 0 : dmmv_pick_rpw(l.ffn_gate_t, D.dim, (int)l.ffn, w.n_groups, w.nt, true);
-    if (!(mq ? launch_mmq(l.ffn_gate_t, 16, true, p, st) : launch_dmmv(l.ffn_gate_t, w.nt, true, p, st)))
+    if (!gu_self && !(mq ? launch_mmq(l.ffn_gate_t, 16, true, p, st) : launch_dmmv(l.ffn_gate_t, w.nt, true, p, st)))
         return fail(LOOMHIP_ERR_ARG, "token_frame: gate/up matvec declined");
+    if (n == 1 && frame_self(l.ffn_down_t, l.ffn_down, nullptr, D.dim, (int)l.ffn, w, w.act, nullptr, 0.0f,
+                                          w.x, 1, st, LOOMHIP_KT_DENSE))
+        return LOOMHIP_OK;
     launch_quant_act(l.ffn_down_t, w.act, (int)l.ffn, (int)l.ffn, (int)n, w.qa_ffn, st);
     if (!frame_matvec(l.ffn_down_t, l.ffn_down, D.dim, (int)l.ffn, w, n, w.qa_ffn, w.x, 1, st, LOOMHIP_KT_DENSE, true))
         return fail(LOOMHIP_ERR_ARG, "token_frame: down matvec declined");

@@ -62,9 +62,11 @@ struct DmmvSegParams {
     int n_seg;
 };
 bool launch_dmmv_seg(int nt, DmmvSegParams sp, hipStream_t st);
-// The same for one vector with the PARITY rmsnorm of x (norm weights norm_w)
-// computed by the launch itself; false = not served.
-bool launch_norm_seg(DmmvSegParams sp, const float *x, const float *norm_w, float eps, hipStream_t st);
+// The same, and a fused pair (base.w2), for groups of one f32 vector each that
+// the launch quantizes itself; norm_w: one group, the PARITY rmsnorm of x
+// applied first.  False = not served (nothing launched).
+bool launch_dmmv_self(bool fused, DmmvSegParams sp, const float *x, int x_stride, const float *norm_w, float eps,
+                      hipStream_t st);
 
 void note_launch();
 // Event timing around tagged launches (LOOMHIP_KT_*); -1 when disabled.

@@ -1101,8 +1101,8 @@ int loomhip_mla_token_frame(const loomhip_mla_layer_desc *descs, size_t n_layers
         const Dev &v = dv[li];
         // the attention head (deepseek.zig:860-886)
         if ((rc = rmsnorm_exact_dev(dx, (int)dim, v.attn_norm, fc->eps, normed, 1, st)) ||
-            (rc = matvec_dev_impl(d.wq.type, q, v.wq, normed, 1, H * kd, dim, st)) ||
-            (rc = matvec_dev_impl(d.kv_a.type, kv, v.kv_a, normed, 1, kvr + rope, dim, st)) ||
+            (rc = matvec_dev_impl(d.wq.type, q, v.wq, normed, 1, H * kd, dim, st, true)) ||
+            (rc = matvec_dev_impl(d.kv_a.type, kv, v.kv_a, normed, 1, kvr + rope, dim, st, true)) ||
             (rc = rmsnorm_exact_dev(kv, (int)kvr, v.kv_a_norm, fc->eps, cache_c(li, pos), 1, st)))
             return rc;
         hipLaunchKernelGGL(mla_rope_kernel, dim3((unsigned)(H + 1)), dim3(64), 0, st, q, (int)H, (int)nope, (int)rope,
@@ -1123,7 +1123,7 @@ int loomhip_mla_token_frame(const loomhip_mla_layer_desc *descs, size_t n_layers
         }
     }
     if ((rc = rmsnorm_exact_dev(dx, (int)dim, d_out_norm, fc->eps, normed, 1, st)) ||
-        (rc = matvec_dev_impl(lm_head.type, dlog, d_lm, normed, 1, vocab, dim, st)))
+        (rc = matvec_dev_impl(lm_head.type, dlog, d_lm, normed, 1, vocab, dim, st, true)))
         return rc;
     e = hipMemcpyAsync(logits, dlog, vocab * 4, hipMemcpyDeviceToHost, st);
     if (e == hipSuccess)
@@ -1172,7 +1172,7 @@ int loomhip_mla_layer_cached_dev(const loomhip_mla_attn *a, const float *const *
     const int nd = (int)(n * dim);
     // x += attn_output . heads (deepseek.zig:1044-1046): n matvecs in one
     // launch (bit-identical to one per sequence), then the residual add
-    if ((rc = matvec_dev_impl(attn_out_type, proj, attn_out, heads, n, dim, hv, st)))
+    if ((rc = matvec_dev_impl(attn_out_type, proj, attn_out, heads, n, dim, hv, st, true)))
         return rc;
     hipLaunchKernelGGL(mla_add_kernel, dim3((unsigned)((nd + 255) / 256)), dim3(256), 0, st, x, proj, nd);
     note_launch();

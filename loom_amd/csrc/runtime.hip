@@ -202,9 +202,12 @@ const DmmvGroup *dense_groups(int n, int nt, int *count) {
 
 int pick_nt(int n) { return n >= 8 ? 8 : n >= 4 ? 4 : n >= 2 ? 2 : 1; }
 
-// Quantize n vectors and run the grouped matvec against one plane.
+// Quantize n vectors and run the grouped matvec against one plane.  self: one
+// vector may be quantized by the matvec's own work groups, in one launch.  The
+// seam's host-buffer calls keep the two: their copies dominate, and their
+// callers read the launch count as the proof that both steps ran.
 int matvec_dev_impl(int t, float *out, const void *w, const float *x, size_t n, size_t rows,
-                    size_t cols, hipStream_t st) {
+                    size_t cols, hipStream_t st, bool self) {
     if (n == 0)
         return LOOMHIP_OK;
     if (t == LH_F32) {
@@ -216,6 +219,25 @@ int matvec_dev_impl(int t, float *out, const void *w, const float *x, size_t n, 
         return fail(LOOMHIP_DECLINED, "dmmv: type %d with %zu columns not served", t, cols);
     if (n > IOTA_LEN)
         return fail(LOOMHIP_DECLINED, "dmmv: %zu vectors exceed %d", n, IOTA_LEN);
+    const bool mq = mmq_dense(t, (int)rows, (int)cols, (int)n, false);
+    if (self && n == 1) {
+        int ng = 0;
+        DmmvSegParams sp{};
+        sp.base.groups = dense_groups(1, 1, &ng);
+        if (!sp.base.groups)
+            return fail(LOOMHIP_ERR_HIP, "dense group table");
+        sp.base.cols = (int)cols;
+        sp.base.pair_src = g_ctx.iota;
+        sp.base.pair_dst = g_ctx.iota;
+        sp.base.n_groups = ng;
+        sp.seg[0] = DmmvSeg{(const uint8_t *)w, t, (int)rows, out, 0, 0};
+        sp.n_seg = 1;
+        const int ph = prof_begin(LOOMHIP_KT_DENSE, st);
+        const bool done = launch_dmmv_self(false, sp, x, (int)cols, nullptr, 0.0f, st);
+        prof_end(ph, st);
+        if (done)
+            return LOOMHIP_OK;
+    }
     const size_t qbytes = align16(n * cols) + align16(n * cols / 32 * 4) + align16(n * cols / 16 * 4);
     int rc = g_ctx.act.reserve(qbytes);
     if (rc)
@@ -225,7 +247,6 @@ int matvec_dev_impl(int t, float *out, const void *w, const float *x, size_t n, 
     qa.d = (float *)((char *)g_ctx.act.ptr + align16(n * cols));
     qa.s = (int32_t *)((char *)qa.d + align16(n * cols / 32 * 4));
     launch_quant_act(t, x, (int)cols, (int)cols, (int)n, qa, st);
-    const bool mq = mmq_dense(t, (int)rows, (int)cols, (int)n, false);
     const int nt = mq ? (n > 16 ? 32 : 16) : pick_nt((int)n);
     int ng = 0;
     const DmmvGroup *groups = dense_groups((int)n, nt, &ng);
@@ -412,7 +433,7 @@ int loomhip_matvec_dev(int t, float *out, const void *w, const float *x, size_t 
                        size_t cols, void *stream) {
     if (int rc = require_ready())
         return rc;
-    return matvec_dev_impl(t, out, w, x, n, rows, cols, stream_of(stream));
+    return matvec_dev_impl(t, out, w, x, n, rows, cols, stream_of(stream), true);
 }
 
 int loomhip_dequant_dev(int t, float *out, const void *w, size_t rows, size_t cols, void *stream) {
@@ -451,7 +472,7 @@ int loomhip_matmul(int t, float *out, const uint8_t *w, const float *xs, size_t 
     if (e != hipSuccess)
         return hip_fail(e, "stage x");
     rc = matvec_dev_impl(t, (float *)g_ctx.ostage.ptr, dw, (const float *)g_ctx.xstage.ptr, n, rows,
-                         cols, st);
+                         cols, st, false);
     if (rc)
         return rc;
     e = hipMemcpyAsync(out, g_ctx.ostage.ptr, n * rows * 4, hipMemcpyDeviceToHost, st);

@@ -45,7 +45,7 @@ hipStream_t stream_of(void *s);
 int upload_weights(int t, const void *host, size_t rows, size_t cols, size_t planes, void **dev);
 void clear_weight_cache();
 int matvec_dev_impl(int t, float *out, const void *w, const float *x, size_t n, size_t rows,
-                    size_t cols, hipStream_t st);
+                    size_t cols, hipStream_t st, bool self);
 int pick_nt(int n);
 // Device group table for n vectors in groups of nt against plane 0 (cached per (n, nt)).
 const DmmvGroup *dense_groups(int n, int nt, int *count);
