@@ -1145,6 +1145,232 @@ static bool launch_mmq32(int t, int max_tok, const DmmvParams &p, hipStream_t st
     return true;
 }
 
+// ---- many vectors: a 64-row x 128-vector tile per work group -----------------------
+// Prefill-sized lane groups (Q4_K / Q6_K).  mmw_kernel decodes a row tile's
+// weights once per 16 vectors; here eight waves share one decode per 128.  Each
+// thread turns 32 weights of a block into two int8 digits of scale * quant
+// (128 a + b: Q4_K sc * q <= 945, Q6_K sc * (q - 32) in 14 bits) in LDS, beside
+// the vectors' int8 columns, and each wave forms 32 rows x 32 vectors with
+// unmasked MFMAs: isum = 128 sum(a x) + sum(b x), exact in any order; Q4_K's mins
+// on one f16 MFMA, as in mmw_kernel.  No multiply per (vector, scale group) is
+// left.  Blocks are taken in order, each output one f32 register -- the
+// reference's `acc += r`.  The LDS (154 KB, one work group per CU) holds two
+// blocks: one is decoded while the other is multiplied and the third's loads
+// are in flight, one barrier per block; the two waves of a SIMD run decode
+// and multiply in opposite order (3% over the same order).
+// Bound by issue, ~4800 cycles of a SIMD per block: 2 x (36 MFMAs at 16, 280
+// VALU ops at ~4), the rest LDS reads and waits.  Q4_K 4096 x 2048 at 512 vectors
+// 30.2 -> 23.5 us, Q6_K 33.8 -> 21.8; 4096 x 8192 at 512 99 -> 71 and 157 -> 64.  A
+// 32 x 64 tile (two groups per CU) took 33.2 / 32.2 at 4096 x 2048.
+constexpr int MMP_R = 64, MMP_T = 128, MMP_W = 8, MMP_ROW = 256 + 16;
+struct MmpLds {
+    int8_t wh[MMP_R * MMP_ROW], wl[MMP_R * MMP_ROW]; // digits, value order
+    int8_t x[MMP_T * MMP_ROW];
+    _Float16 bs[MMP_T * 20]; // 16 sums per vector
+    _Float16 mn[MMP_R * 10]; // 8 mins per row
+    float d[MMP_R * 2];      // (d, dmin) per row
+    float xd[MMP_T];
+};
+
+template <int T>
+__global__ __launch_bounds__(64 * MMP_W, 2) void mmp_kernel(DmmvParams p) {
+    extern __shared__ __align__(16) uint8_t sh[];
+    constexpr bool K4 = T == LH_Q4_K;
+    MmpLds *buf = (MmpLds *)sh;
+    const int n = p.ident_n, cols = p.cols, nb = cols / 256, tid = threadIdx.x;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), ln = tid & 63, r16 = ln & 15, q4 = ln >> 4;
+    const int row0 = (int)blockIdx.x * MMP_R, tok0 = (int)blockIdx.y * MMP_T;
+    // this thread's share of a block: 16 bytes of quants of one row, four 16-byte
+    // pieces of the vectors' columns, four sums
+    const int wr = tid >> 3, wc = tid & 7;
+    const size_t U = (size_t)p.rows * nb, wrow = (size_t)min(row0 + wr, p.rows - 1) * nb;
+    const int8_t *xp[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+        xp[i] = p.xq + (size_t)p.pair_src[min(tok0 + 32 * i + (tid >> 4), n - 1)] * cols + 16 * (tid & 15);
+    const int32_t *sp = p.xs + (size_t)p.pair_src[min(tok0 + (tid >> 2), n - 1)] * (cols / 16) + 4 * (tid & 3);
+    const float *dp = p.xd + (size_t)p.pair_src[min(tok0 + (tid & (MMP_T - 1)), n - 1)] * nb;
+    struct Raw {
+        mmq_i4 q, h, s; // quants; Q4_K the header, Q6_K the high bits; the vector's sums (Q4_K) or the scales (Q6_K)
+        mmq_i4 x[4];
+        float xd;
+        uint32_t d;
+    } raw;
+    auto fetch = [&](int b) {
+        const size_t u = wrow + b;
+        if constexpr (K4) {
+            raw.q = *(const mmq_i4 *)(p.w + u * 144 + 16 + 16 * wc);
+            raw.h = *(const mmq_i4 *)(p.w + u * 144);
+            raw.s = *(const mmq_i4 *)(sp + 16 * b);
+        } else {
+            raw.q = *(const mmq_i4 *)(p.w + u * 128 + 16 * wc);
+            raw.h = *(const mmq_i4 *)(p.w + U * 128 + u * 64 + 32 * (wc >> 2) + 16 * (wc & 1));
+            raw.s = *(const mmq_i4 *)(p.w + U * 192 + u * 16);
+            raw.d = *(const uint16_t *)(p.w + U * 208 + u * 2);
+        }
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+            raw.x[i] = *(const mmq_i4 *)(xp[i] + 256 * b);
+        raw.xd = dp[b];
+    };
+    auto decode = [&](MmpLds &l) {
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+            *(mmq_i4 *)(l.x + (32 * i + (tid >> 4)) * MMP_ROW + 16 * (tid & 15)) = raw.x[i];
+        if (tid < MMP_T)
+            l.xd[tid] = raw.xd;
+        mmq_i4 h0, l0, h1, l1; // the 16 low-nibble values' digits, the 16 high-nibble ones'
+        int k0, k1;            // their first value's place in the block
+        if constexpr (K4) {
+            const uint32_t a = raw.h[1], m = raw.h[2], c = raw.h[3];
+            const int p2 = wc >> 1; // groups 2 p2, 2 p2 + 1
+            const uint32_t scv = p2 < 2 ? a & 0x3F3F3F3Fu : (c & 0x0F0F0F0Fu) | ((a >> 2) & 0x30303030u);
+            const uint32_t scs = scv >> (16 * (p2 & 1));
+            const short s0 = (short)(scs & 0xFF), s1 = (short)((scs >> 8) & 0xFF);
+            const mmq_s2 z2 = {0, 0};
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                int hi, lo;
+                q6k_digits((uint32_t)raw.q[e] & 0x0F0F0F0Fu, mmq_s2{s0, s0}, z2, hi, lo);
+                h0[e] = hi, l0[e] = lo;
+                q6k_digits(((uint32_t)raw.q[e] >> 4) & 0x0F0F0F0Fu, mmq_s2{s1, s1}, z2, hi, lo);
+                h1[e] = hi, l1[e] = lo;
+            }
+            k0 = 64 * p2 + 16 * (wc & 1);
+            k1 = k0 + 32;
+            // min of group wc, the row's (d, dmin), the vector's sums
+            const uint32_t mv = wc < 4 ? m & 0x3F3F3F3Fu : ((c >> 4) & 0x0F0F0F0Fu) | ((m >> 2) & 0x30303030u);
+            l.mn[10 * wr + wc] = (_Float16)(unsigned short)((mv >> (8 * (wc & 3))) & 0xFF);
+            if (wc == 0) {
+                l.d[2 * wr] = half_bits_to_float((uint32_t)raw.h[0] & 0xffff);
+                l.d[2 * wr + 1] = half_bits_to_float((uint32_t)raw.h[0] >> 16);
+            }
+            *(mmq_h4 *)(l.bs + 20 * (tid >> 2) + 4 * (tid & 3)) =
+                mmq_h4{(_Float16)(short)raw.s[0], (_Float16)(short)raw.s[1], (_Float16)(short)raw.s[2],
+                       (_Float16)(short)raw.s[3]};
+        } else {
+            const int h = wc >> 2, qa = (wc >> 1) & 1, r = wc & 1; // quarters qa and qa + 2 of half h, run r
+            const uint32_t s01 = h ? (uint32_t)raw.s[2] : (uint32_t)raw.s[0]; // scales 8h .. 8h + 3
+            const uint32_t s23 = h ? (uint32_t)raw.s[3] : (uint32_t)raw.s[1]; // 8h + 4 .. 8h + 7
+            const short s0 = (short)(int8_t)((s01 >> (8 * (2 * qa + r))) & 0xFF);
+            const short s1 = (short)(int8_t)((s23 >> (8 * (2 * qa + r))) & 0xFF);
+            mmq_s2 o0 = mmq_s2{s0, s0} * (short)-32, o1 = mmq_s2{s1, s1} * (short)-32;
+            asm("" : "+v"(o0), "+v"(o1));
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const uint32_t ql = (uint32_t)raw.q[e], qh = (uint32_t)raw.h[e];
+                int hi, lo;
+                q6k_digits((ql & 0x0F0F0F0Fu) | (((qh >> (2 * qa)) & 0x03030303u) << 4), mmq_s2{s0, s0}, o0, hi, lo);
+                h0[e] = hi, l0[e] = lo;
+                q6k_digits(((ql >> 4) & 0x0F0F0F0Fu) | (((qh >> (4 + 2 * qa)) & 0x03030303u) << 4), mmq_s2{s1, s1}, o1,
+                           hi, lo);
+                h1[e] = hi, l1[e] = lo;
+            }
+            k0 = 128 * h + 32 * qa + 16 * r;
+            k1 = k0 + 64;
+            if (wc == 0)
+                l.d[2 * wr] = half_bits_to_float(raw.d);
+        }
+        *(mmq_i4 *)(l.wh + wr * MMP_ROW + k0) = h0;
+        *(mmq_i4 *)(l.wl + wr * MMP_ROW + k0) = l0;
+        *(mmq_i4 *)(l.wh + wr * MMP_ROW + k1) = h1;
+        *(mmq_i4 *)(l.wl + wr * MMP_ROW + k1) = l1;
+    };
+    const int wrow0 = 32 * (wave & 1), wtok0 = 32 * (wave >> 1); // this wave's 32 x 32
+    float acc[2][2][4] = {};
+    const mmq_i4 z = {0, 0, 0, 0};
+    auto multiply = [&](const MmpLds &l) {
+        mmq_i4 ah[2][2], al[2][2];
+        mmq_f4 ms[2][2];
+        if constexpr (K4) {
+            mmq_h4 bs[2], mn[2];
+#pragma unroll
+            for (int i = 0; i < 2; i++) {
+                bs[i] = *(const mmq_h4 *)(l.bs + 20 * (wtok0 + 16 * i + r16) + 4 * q4);
+                const _Float16 *m = l.mn + 10 * (wrow0 + 16 * i + r16) + 2 * q4;
+                mn[i] = mmq_h4{m[0], m[0], m[1], m[1]};
+            }
+#pragma unroll
+            for (int t = 0; t < 2; t++)
+#pragma unroll
+                for (int r = 0; r < 2; r++)
+                    ms[t][r] = __builtin_amdgcn_mfma_f32_16x16x16f16(bs[t], mn[r], mmq_f4{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
+        }
+#pragma unroll
+        for (int s = 0; s < 4; s++) {
+            mmq_i4 xa[2], bh[2], bl[2];
+#pragma unroll
+            for (int i = 0; i < 2; i++) {
+                xa[i] = *(const mmq_i4 *)(l.x + (wtok0 + 16 * i + r16) * MMP_ROW + 64 * s + 16 * q4);
+                bh[i] = *(const mmq_i4 *)(l.wh + (wrow0 + 16 * i + r16) * MMP_ROW + 64 * s + 16 * q4);
+                bl[i] = *(const mmq_i4 *)(l.wl + (wrow0 + 16 * i + r16) * MMP_ROW + 64 * s + 16 * q4);
+            }
+#pragma unroll
+            for (int t = 0; t < 2; t++)
+#pragma unroll
+                for (int r = 0; r < 2; r++) {
+                    ah[t][r] = __builtin_amdgcn_mfma_i32_16x16x64_i8(xa[t], bh[r], s ? ah[t][r] : z, 0, 0, 0);
+                    al[t][r] = __builtin_amdgcn_mfma_i32_16x16x64_i8(xa[t], bl[r], s ? al[t][r] : z, 0, 0, 0);
+                }
+        }
+#pragma unroll
+        for (int r = 0; r < 2; r++) {
+            const float2 d = *(const float2 *)(l.d + 2 * (wrow0 + 16 * r + r16));
+#pragma unroll
+            for (int t = 0; t < 2; t++) {
+                const float4 v = *(const float4 *)(l.xd + wtok0 + 16 * t + 4 * q4);
+                const float xd[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    const float is = (float)((ah[t][r][i] << 7) + al[t][r][i]);
+                    if constexpr (K4) {
+                        // xb.d * (d * f32(isum) - dmin * f32(min_isum))  (ggml.zig:1016-1017)
+                        const float aa = d.x * is, bb = d.y * ms[t][r][i];
+                        acc[t][r][i] = acc[t][r][i] + xd[i] * (aa - bb);
+                    } else {
+                        // xb.d * dec.d * f32(isum)  (ggml.zig:1019)
+                        const float s = xd[i] * d.x;
+                        acc[t][r][i] = acc[t][r][i] + s * is;
+                    }
+                }
+            }
+        }
+    };
+    fetch(0);
+    decode(buf[0]);
+    fetch(min(1, nb - 1));
+    lds_barrier();
+    for (int b = 0; b < nb; b++) {
+        if (wave >= MMP_W / 2)
+            multiply(buf[b & 1]);
+        if (b + 1 < nb) { // the other buffer's readers passed the last barrier
+            decode(buf[(b + 1) & 1]);
+            fetch(min(b + 2, nb - 1)); // past the last block: the last one again, not used
+        }
+        if (wave < MMP_W / 2)
+            multiply(buf[b & 1]);
+        lds_barrier();
+    }
+#pragma unroll
+    for (int t = 0; t < 2; t++)
+#pragma unroll
+        for (int r = 0; r < 2; r++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const int tok = tok0 + wtok0 + 16 * t + 4 * q4 + i, row = row0 + wrow0 + 16 * r + r16;
+                if (tok >= n || row >= p.rows)
+                    continue;
+                float *o = p.out + (size_t)tok * p.out_stride + row;
+                *o = p.accumulate ? *o + acc[t][r][i] : acc[t][r][i];
+            }
+}
+
+template <int T>
+static void mmp_launch_t(const DmmvParams &p, hipStream_t st) {
+    const dim3 grid((p.rows + MMP_R - 1) / MMP_R, (p.ident_n + MMP_T - 1) / MMP_T);
+    hipLaunchKernelGGL(mmp_kernel<T>, grid, dim3(64 * MMP_W), 2 * sizeof(MmpLds), st, p);
+}
+
 // ---- Q8_0 / Q4_0 streamed in block order ------------------------------------------
 // mmw_kernel's shape for 32-value blocks: a wave owns 16 rows for up to 16
 // tokens of a group and walks them in units of 8 blocks (256 columns),
@@ -1512,6 +1738,21 @@ static bool lanes_streamed(int t, int rows, int cols, int n, bool fused) {
            lane_pairs(rows, n) >= (fused ? MMW_MIN_WAVES_FUSED : MMW_MIN_WAVES);
 }
 
+// Lane groups that fill mmp_kernel's 64 x 128 tiles and whole rounds of the
+// chip's 256 CUs with them: the pairs that the launch holds over those that its
+// rounds could (256 tiles of 32).  A round costs mmp_kernel the same however few
+// of its CUs work; Q4_K breaks even at ~3/4, Q6_K at ~3/5.  Measured, us, streamed /
+// this: Q4_K 4096 x 2048 at 256 (half a round) 18.7 / 21.8, 8192 x 1024 at 256 (one)
+// 18.5 / 14.7, 16384 x 2048 at 192 (3/4) 38.4 / 40.6, at 256 (two rounds) 48.0 / 41.1;
+// Q6_K 20.1 / 20.0, 20.1 / 13.9, 43.9 / 37.1, 55.2 / 37.6.
+static bool lanes_tiled(int t, int rows, int cols, int n) {
+    if (!is_k(t) || !mmw_shape(t, rows, cols, false))
+        return false;
+    const long tiles = (long)((rows + MMP_R - 1) / MMP_R) * ((n + MMP_T - 1) / MMP_T);
+    const long room = (tiles + 255) / 256 * 256 * (MMP_R / 16) * (MMP_T / 16);
+    return t == LH_Q4_K ? lane_pairs(rows, n) * 5 >= room * 4 : lane_pairs(rows, n) * 3 >= room * 2;
+}
+
 // n vectors against one [rows][cols] matrix (or a fused pair): whether the
 // matrix cores take them from the dot4 matvec.  By type and size, us per
 // launch, dot4 / matrix cores: Q4_K 4096 x 4096 at 5 vectors 11.4 / 9.1,
@@ -1624,6 +1865,11 @@ bool launch_mmq(int t, int max_tok, bool fused, const DmmvParams &p, hipStream_t
             fused ? mmw32_launch_t<LH_Q8_0, true>(p, st) : mmw32_launch_t<LH_Q8_0, false>(p, st);
         else
             fused ? mmw32_launch_t<LH_Q4_0, true>(p, st) : mmw32_launch_t<LH_Q4_0, false>(p, st);
+        note_launch();
+        return true;
+    }
+    if (p.ident_n > 0 && !fused && lanes_tiled(t, p.rows, p.cols, p.ident_n)) {
+        t == LH_Q4_K ? mmp_launch_t<LH_Q4_K>(p, st) : mmp_launch_t<LH_Q6_K>(p, st);
         note_launch();
         return true;
     }

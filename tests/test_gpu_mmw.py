@@ -1,5 +1,5 @@
 """GPU parity of the matrix-core matmul that streams a row's blocks in order
-(mmw_kernel, mmq.hip): bit-exact against per-vector oracle matvecs at the edges
+(mmw_kernel, mmq.hip) and of the one with 64 x 128 tiles (mmp_kernel): bit-exact against per-vector oracle matvecs at the edges
 of its row tiles (16 rows, 64 per work group), token sets (8) and groups (16,
 32), block counts (odd and even, with the tokens' rows staged in LDS up to
 2048 columns and not beyond), and at the extreme integers of its f16 mins and
@@ -45,11 +45,12 @@ def test_streamed_matmul_edges(be, oracle, t, rows, cols, n):
 
 
 @pytest.mark.parametrize("t", [Q4_K, Q6_K])
-def test_streamed_matmul_extreme_integers(be, oracle, t):
+@pytest.mark.parametrize("n", [16, 128])
+def test_streamed_matmul_extreme_integers(be, oracle, t, n):
     """Every quant, scale and min at an end of its range against activations of
     one sign: the largest block integers (Q4_K 8 * 63 * 15 * 32 * 127 and the
     mins' 16 * 63 * 2032, Q6_K 128 * 32 * 256 * 127) through every exact step."""
-    rows, cols, n = 16384, 512, 16
+    rows, cols = 16384, 512
     rng = np.random.default_rng(5 + t)
     raw = npref.pinned_scale_blocks(t, rows, cols, rng)
     b = raw.reshape(-1, 144 if t == Q4_K else 210)
@@ -65,6 +66,18 @@ def test_streamed_matmul_extreme_integers(be, oracle, t):
     xs = np.ones((n, cols), np.float32)
     xs[1::2] = -3.0
     xs[2::4, ::2] = -1.0
+    _check(be, oracle, t, raw, xs, rows, cols)
+
+
+# tiles of 64 rows x 128 vectors that fill a round of 256 CUs: full tiles, one row
+# and one vector short of / past an edge, one to three blocks, a partial second round
+@pytest.mark.parametrize("t", [Q4_K, Q6_K])
+@pytest.mark.parametrize("rows,cols,n", [(8192, 512, 256), (8192 - 65, 768, 255), (4096 - 63, 256, 511),
+                                         (14000, 512, 255), (16384 + 8192, 256, 257 - 4)])
+def test_tiled_matmul_edges(be, oracle, t, rows, cols, n):
+    rng = np.random.default_rng(rows + cols + n + t)
+    raw = npref.pinned_scale_blocks(t, rows, cols, rng)
+    xs = np.stack([oracle.normal(cols, 100 * n + k, 0.0, float(k % 5 + 1)) for k in range(n)])
     _check(be, oracle, t, raw, xs, rows, cols)
 
 
