@@ -7,11 +7,18 @@
 // The integer part of every block dot runs on the int8 MFMAs: the activations
 // of 16 tokens are the A rows, 16 weight rows the B columns (Q4_K:
 // v_mfma_i32_16x16x64_i8 over a 64-value quant span; Q6_K: the same MFMA
-// over four 16-value runs, one run per MFMA).  Integer dots are exact in
-// any order, so isum = sum sc * dot and msum = sum mn * bsum are the
-// reference's integers; the f32 tail per (token, row, super-block) is the
-// reference's expression, and each output sums its blocks in block order
-// from LDS.
+// over four 16-value runs, one run per MFMA, or over two int8 digits of
+// scale * quant).  Integer dots are exact in any order, so isum = sum sc * dot
+// and msum = sum mn * bsum are the reference's integers; the f32 tail per
+// (token, row, super-block) is the reference's expression, and each output
+// sums its blocks in block order.
+//
+// Three forms, chosen in launch_mmq by what fills the chip:
+//   one-shot (mmq_kernel, mmq_seg_kernel, mmq32_kernel): a row tile's blocks
+//     spread over the waves of a work group, summed from LDS -- small matrices;
+//   streamed (mmw_kernel, mmw32_kernel): a wave takes a row tile and walks its
+//     blocks in order, the sums in registers -- expert groups, large matrices;
+//   tiled (mmp_kernel): 64 rows x 128 vectors per work group -- prefill sizes.
 //
 // Lane l of a wave: weight row l % 16 of its 16-row tile, k-quarter l / 16;
 // the result lane l holds tokens 4*(l/16) .. +3 of that row.
@@ -1738,6 +1745,18 @@ static bool lanes_streamed(int t, int rows, int cols, int n, bool fused) {
            lane_pairs(rows, n) >= (fused ? MMW_MIN_WAVES_FUSED : MMW_MIN_WAVES);
 }
 
+// Expert groups of K-quants with fewer (group, row tile, matrix) streams than
+// this take the one-shot kernel: the groups the launch has room for, a little
+// over nine streams per CU.  Measured, us per layer, one-shot / streamed gate/up
+// and down: 1024 x 512 x 32 top-4 Q4_K + Q6_K at 16 tokens (2304 streams each)
+// 32.3 / 34.4, at 19 33.9 / 35.6, at 24 (2432) 37.2 / 37.0, at 128 (4096) 49.7 /
+// 45.9; 2048 x 768 x 128 top-8 at 10 (8160 and 10880) 58.1 / 52.4.  The 32-value
+// blocks' one-shot form is slower at every size (63 / 41 at 24 tokens).
+constexpr long MMW_MIN_GROUP_STREAMS = 2400;
+static bool groups_few(int t, int rows, int n_groups, bool fused) {
+    return is_k(t) && (long)n_groups * ((rows + 15) / 16) * (fused ? 2 : 1) < MMW_MIN_GROUP_STREAMS;
+}
+
 // Lane groups that fill mmp_kernel's 64 x 128 tiles and whole rounds of the
 // chip's 256 CUs with them: the pairs that the launch holds over those that its
 // rounds could (256 tiles of 32).  A round costs mmp_kernel the same however few
@@ -1780,10 +1799,10 @@ bool mmq_dense(int t, int rows, int cols, int n, bool fused) {
 // The expert matmuls of n tokens: whether they run on the matrix cores in
 // groups of 16.  By type and expert size, us per layer with the dot4 / matrix
 // core matmuls, Zipf-skewed router: Q4_K + Q6_K 2048 x 768 x 128 at 5 tokens
-// 48.8 / 46.4 (uniform 58.3 / 56.8), 1024 x 512 x 32 at 8 32.4 / 32.9, at 10
-// 35.2 / 34.0; Q8_0 2048 x 768 at 8 66.7 / 61.7 (uniform 79.3 / 86.7), at 12
-// 90.5 / 66.2 (113 / 97), Q4_0 at 12 76.3 / 57.5; 7168 x 2048 x 16 at 5 Q8_0
-// 183 / 150, Q4_0 142 / 116; Q8_0 1024 x 512 x 32 at 15 35.2 / 40.1.
+// 48.8 / 46.4 (uniform 58.3 / 56.8), 1024 x 512 x 32 at 10 35.2 / 32.1; Q8_0
+// 2048 x 768 at 8 66.7 / 61.7 (uniform 79.3 / 86.7), at 12 90.5 / 66.2 (113 /
+// 97), Q4_0 at 12 76.3 / 57.5; 7168 x 2048 x 16 at 5 Q8_0 183 / 150, Q4_0 142 /
+// 116; Q8_0 1024 x 512 x 32 at 15 35.2 / 40.1.
 static int experts_min(int t, size_t size) {
     if (is_k(t))
         return size >= 1500000 ? 5 : 10;
@@ -1845,7 +1864,7 @@ bool launch_mmq_seg(DmmvSegParams sp, hipStream_t st) {
 }
 
 // Groups of at most max_tok (<= 32) tokens (with p.ident_n: max_tok sets
-// the group size); p.rpw is unused.  Expert groups (<= 16 tokens) stream.
+// the group size); p.rpw is unused.
 bool launch_mmq(int t, int max_tok, bool fused, const DmmvParams &p, hipStream_t st) {
     if (p.rows < 1 || max_tok < 1 || max_tok > 32)
         return false;
@@ -1854,7 +1873,8 @@ bool launch_mmq(int t, int max_tok, bool fused, const DmmvParams &p, hipStream_t
     const bool oneshot = mmq_oneshot(t, p.cols, max_tok, fused);
     const bool stream = p.ident_n > 0 ? lanes_streamed(t, p.rows, p.cols, p.ident_n, fused) ||
                                             (!oneshot && mmw_shape(t, p.rows, p.cols, fused))
-                                      : max_tok <= 16 && mmw_shape(t, p.rows, p.cols, fused);
+                                      : max_tok <= 16 && mmw_shape(t, p.rows, p.cols, fused) &&
+                                            !(oneshot && groups_few(t, p.rows, p.n_groups, fused));
     if (!stream && !oneshot)
         return false;
     const int mt = max_tok > 16 ? 2 : 1;

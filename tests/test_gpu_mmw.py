@@ -33,7 +33,7 @@ def _check(be, oracle, t, raw, xs, rows, cols):
     assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
 
 
-# (row tiles) x (groups of 16 vectors) >= 1024 takes the streamed kernel
+# (row tiles) x (groups of 16 vectors) >= 768 takes the streamed kernel
 @pytest.mark.parametrize("t", [Q4_K, Q6_K])
 @pytest.mark.parametrize("rows,cols,n", [(16384 + 1, 256, 16), (8192 + 15, 768, 17), (8192 + 49, 512, 25),
                                          (8192, 2048, 32), (8192 + 16, 2304, 24), (16384 + 33, 2816, 16)])
@@ -132,10 +132,12 @@ def test_matmul_from_five_vectors(be, oracle, t, rows, cols, n):
 
 
 @pytest.mark.parametrize("t,dim,ffn,n", [(Q8_0, 288, 96, 21), (Q4_0, 544, 288, 40), (Q8_0, 2080, 768, 12),
-                                         (Q4_0, 1024, 1536, 13), (Q4_K, 512, 256, 10), (Q4_K, 2304, 768, 5)])
+                                         (Q4_0, 1024, 1536, 13), (Q4_K, 512, 256, 10), (Q4_K, 2304, 768, 5),
+                                         (Q4_K, 2304, 3072, 17), (Q4_K, 4352, 1536, 17)])
 def test_moe_layer_streamed_experts(be, oracle, t, dim, ffn, n):
-    """The routed layer with its expert matmuls streamed in groups of 16 for
-    every type: ids, gates and output bits against lo_moe_batch_union."""
+    """The routed layer with its expert matmuls in groups of 16 for every type
+    (streamed; Q4_K gate/up streamed from 2304 x 3072 on, down from 4352 x
+    1536, one-shot below): ids, gates and output bits against lo_moe_batch_union."""
     import torch
     from test_gpu_moe import _dev_layer, make_layer
 
