@@ -65,7 +65,7 @@ MFMA_I8_OPS = 2 * 16 * 16 * 64
 FFN = 768
 # The grouped expert launches at 16+ tokens and the kernels that serve them
 # (config 4: Q4_K gate/up over 2048 columns, Q6_K down over 768)
-MOE_GEMM_KERNELS = {"gate_up": "lh::mmqs_kernel<true, 8>", "down": "lh::mmq_kernel<14, 1, false, 1>"}
+MOE_GEMM_KERNELS = {"gate_up": "lh::mmw_kernel<12, 1, true, true, 3>", "down": "lh::mmw_kernel<14, 1, false, true, 4>"}
 # Largest per-step logit max-rel of FAST numerics against the CPU path at the
 # 4096-token context (32 lanes), measured by the GPU parity test named in the
 # output line.
@@ -304,10 +304,10 @@ def moe_gemm(r, b, ctx):
     the bf16 and int8 dense peaks and against the attainable min(int8 peak,
     AI x HBM peak), AI = useful ops / the launch's algorithmic bytes.  Issued
     = the MFMAs the kernels run for this layer's groups (experts' tokens in
-    groups of up to 16): gate/up per (group, 16-row tile, super-block) one
-    set of 8 MFMAs per matrix per 8 tokens (4 dot + 4 mins, A rows = (token,
-    group)), down 16 per (group, 16-row tile, super-block) (one per 16-value
-    run); beside it the count rocprofv3 measured, and the same rates over
+    groups of up to 16): gate/up per (group, 16-row tile, super-block) 4 int8
+    MFMAs per matrix per 8 tokens (A rows = (token, group); the mins run on
+    one f16 MFMA, not counted), down 8 per (group, 16-row tile, super-block)
+    (two int8 digits of scale * quant over four 64-value spans); beside it the count rocprofv3 measured, and the same rates over
     the committed rocprof duration."""
     pairs = b * TOP_K
     out = {}
@@ -318,9 +318,9 @@ def moe_gemm(r, b, ctx):
         avg_s = s["ms"] / s["count"] / 1e3
         useful = (2 if tag == "gate_up" else 1) * 2 * pairs * FFN * DIM
         if tag == "gate_up":
-            issued = r["sets8"] * 2 * 8 * (FFN // 16) * (DIM // 256) * MFMA_I8_OPS
+            issued = r["sets8"] * 2 * 4 * (FFN // 16) * (DIM // 256) * MFMA_I8_OPS
         else:
-            issued = r["groups"] * 16 * (DIM // 16) * (FFN // 256) * MFMA_I8_OPS
+            issued = r["groups"] * 8 * (DIM // 16) * (FFN // 256) * MFMA_I8_OPS
         byts = per_launch_bytes(tag, b, ctx, r["distinct"])
         ai = useful / byts
         attain = min(PEAK_INT8_OPS, ai * HBM_PEAK_GBS * 1e9)
@@ -576,8 +576,7 @@ def bench_moe_layer(args):
                     "distinct_experts": round(dist, 1), "bytes": int(byts), "GBs": round(gbs, 1),
                     "hbm_frac": round(gbs / HBM_PEAK_GBS, 4), "flops": flops,
                     "TFLOPs": round(flops / (ms / 1e3) / 1e12, 2),
-                    "path": "decode kernels" if b <= 4 else "grouped matrix-core matmul" if b >= 16 else
-                            "grouped matvec"})
+                    "path": "decode kernels" if b <= 4 else "grouped matrix-core matmul"})
         log(f"moe layer batch {b}: {ms * 1e3:.2f} us, {dist:.1f} distinct experts, {gbs:.0f} GB/s")
     return {"metric": "one MoE layer: us per layer and GB/s of distinct expert bytes (config 3)", "n_gpus": 1,
             "peak_GBs": HBM_PEAK_GBS, "data": "synthetic", "dtype": "int8",
