@@ -307,8 +307,9 @@ def moe_gemm(r, b, ctx):
     groups of up to 16): gate/up per (group, 16-row tile, super-block) 4 int8
     MFMAs per matrix per 8 tokens (A rows = (token, group); the mins run on
     one f16 MFMA, not counted), down 8 per (group, 16-row tile, super-block)
-    (two int8 digits of scale * quant over four 64-value spans); beside it the count rocprofv3 measured, and the same rates over
-    the committed rocprof duration."""
+    (two int8 digits of scale * quant over four 64-value spans); beside it the
+    count rocprofv3 measured, and the same rates over the committed rocprof
+    duration."""
     pairs = b * TOP_K
     out = {}
     for tag, kern in MOE_GEMM_KERNELS.items():

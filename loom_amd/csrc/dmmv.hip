@@ -209,8 +209,10 @@ __global__ __launch_bounds__(256) void dmmv_seg_kernel(DmmvSegParams sp) {
 // (the sequential sum of the squares, 4 waves), every work group for itself --
 // the attention norm with q, k and v, the FFN norm with gate and up.  The
 // stories15M token (6 layers, dim 288): 66 -> 42 launches, 292 -> 230 us; a
-// matvec call from Python 10.8 -> 7.4 us at 768 x 2048.  Same values as norm_quant_kernel / quant_act_kernel followed by dmmv_seg_kernel
-// or dmmv_kernel.
+// matvec call from Python 10.8 -> 7.4 us at 768 x 2048 (the kernel alone 6.1 to
+// 6.7 us up to 2048 x 2048, where the two took 4.6 and 4.7 to 5.1).  Same values
+// as norm_quant_kernel / quant_act_kernel followed by dmmv_seg_kernel or
+// dmmv_kernel.
 constexpr int NSEG_MAX_DIM = 4096;
 constexpr int NSEG_XV = norm_xv(NSEG_MAX_DIM, 4);
 

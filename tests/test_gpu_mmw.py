@@ -1,9 +1,10 @@
 """GPU parity of the matrix-core matmul that streams a row's blocks in order
-(mmw_kernel, mmq.hip) and of the one with 64 x 128 tiles (mmp_kernel): bit-exact against per-vector oracle matvecs at the edges
-of its row tiles (16 rows, 64 per work group), token sets (8) and groups (16,
-32), block counts (odd and even, with the tokens' rows staged in LDS up to
-2048 columns and not beyond), and at the extreme integers of its f16 mins and
-two-digit scales.  Runs on the MI355X box only."""
+(mmw_kernel, mmq.hip) and of the one with 64 x 128 tiles (mmp_kernel):
+bit-exact against per-vector oracle matvecs at the edges of its row tiles (16
+rows, 64 per work group), token sets (8) and groups (16, 32), block counts (odd
+and even, with the tokens' rows staged in LDS up to 2048 columns and not
+beyond), and at the extreme integers of its f16 mins and two-digit scales.
+Needs the GPU."""
 import numpy as np
 import pytest
 
