@@ -211,7 +211,8 @@ size_t loomhip_materialize_arenas(void);
 
 /* ---- device-resident hot path ------------------------------------------- */
 
-/* out[n][rows] = W . x_k for n activation vectors x[n][cols] (device f32). */
+/* out[n][rows] = W . x_k for n activation vectors x[n][cols] (device f32).
+ * For a quantized type out may overlap x. */
 int loomhip_matvec_dev(int t, float *out, const void *w, const float *x, size_t n, size_t rows,
                        size_t cols, void *stream);
 int loomhip_dequant_dev(int t, float *out, const void *w, size_t rows, size_t cols, void *stream);

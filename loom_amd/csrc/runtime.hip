@@ -202,8 +202,14 @@ const DmmvGroup *dense_groups(int n, int nt, int *count) {
 
 int pick_nt(int n) { return n >= 8 ? 8 : n >= 4 ? 4 : n >= 2 ? 2 : 1; }
 
+static bool overlap(const void *a, size_t na, const void *b, size_t nb) {
+    return (uintptr_t)a < (uintptr_t)b + nb && (uintptr_t)b < (uintptr_t)a + na;
+}
+
 // Quantize n vectors and run the grouped matvec against one plane.  self: one
-// vector may be quantized by the matvec's own work groups, in one launch.  The
+// vector may be quantized by the matvec's own work groups, in one launch; not
+// where out overlaps x, which every one of those work groups reads while
+// others store (the two launches read all of x before any store).  The
 // seam's host-buffer calls keep the two: their copies dominate, and their
 // callers read the launch count as the proof that both steps ran.
 int matvec_dev_impl(int t, float *out, const void *w, const float *x, size_t n, size_t rows,
@@ -220,7 +226,7 @@ int matvec_dev_impl(int t, float *out, const void *w, const float *x, size_t n, 
     if (n > IOTA_LEN)
         return fail(LOOMHIP_DECLINED, "dmmv: %zu vectors exceed %d", n, IOTA_LEN);
     const bool mq = mmq_dense(t, (int)rows, (int)cols, (int)n, false);
-    if (self && n == 1) {
+    if (self && n == 1 && !overlap(out, rows * 4, x, cols * 4)) {
         int ng = 0;
         DmmvSegParams sp{};
         sp.base.groups = dense_groups(1, 1, &ng);

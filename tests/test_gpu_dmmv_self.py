@@ -31,3 +31,32 @@ def test_one_vector_matvec_dev(oracle, t, rows, cols):
     torch.cuda.synchronize()
     want = oracle.matvec(t, raw, x, rows, cols)
     assert np.array_equal(out.cpu().numpy().view(np.uint32), want.view(np.uint32))
+
+
+@pytest.mark.parametrize("t,rows,cols", [(Q4_0, 768, 768), (Q8_0, 2048, 2048), (Q4_K, 2048, 2048), (Q6_K, 2304, 768),
+                                         (Q4_0, 96, 2048)])
+@pytest.mark.parametrize("place", ["same", "tail", "head", "behind"])
+def test_one_vector_matvec_dev_over_its_input(oracle, t, rows, cols, place):
+    """out over x: at the same address, by x's last four elements, by out's
+    last four, and right behind x without overlap.  The launches tell the route:
+    two where the ranges meet (all of x is read before the first store), one
+    where they do not."""
+    import torch
+
+    import loom_amd
+    from loom_amd import backend as be
+
+    loom_amd.init(0)
+    raw = npref.pinned_scale_blocks(t, rows, cols, np.random.default_rng(rows + cols + t))
+    w = be.repack_dev(t, torch.from_numpy(raw).cuda(), rows, cols, 1)
+    x = oracle.normal(cols, rows + cols, 0.0, 1.0)
+    ox, oo = {"same": (0, 0), "tail": (0, cols - 4), "head": (rows - 4, 0), "behind": (0, cols)}[place]
+    buf = torch.zeros(rows + 2 * cols, device="cuda")
+    buf[ox:ox + cols] = torch.from_numpy(x).cuda()
+    out = buf[oo:oo + rows]
+    loom_amd.take_launch_count()
+    assert be.matvec_dev(t, out, w, buf[ox:ox + cols], 1, rows, cols) == loom_amd.OK
+    assert loom_amd.take_launch_count() == (1 if place == "behind" else 2)
+    torch.cuda.synchronize()
+    want = oracle.matvec(t, raw, x, rows, cols)
+    assert np.array_equal(out.cpu().numpy().view(np.uint32), want.view(np.uint32))
