@@ -494,7 +494,7 @@ static int moe_cached(const loomhip_moe_layer_ec &L, loomhip_ec *c, const float 
             gu.rpw = dmmv_pick_rpw(L.gate_t, (int)L.dim, (int)L.ffn, ng, nt, true);
             int ph = prof_begin(LOOMHIP_KT_GATE_UP, st);
             bool ok = launch_dmmv(L.gate_t, nt, true, gu, st);
-            prof_end(ph, st);
+            prof_end(ph, st, ok);
             if (!ok)
                 return tables_done(fail(LOOMHIP_ERR_ARG, "moe_cached: gate/up partials exceed LDS"));
             launch_quant_act(L.down_t, act, (int)L.ffn, (int)L.ffn, np, qa, st);
@@ -515,7 +515,7 @@ static int moe_cached(const loomhip_moe_layer_ec &L, loomhip_ec *c, const float 
             dn.rpw = dmmv_pick_rpw(L.down_t, (int)L.ffn, (int)L.dim, ng, nt, false);
             ph = prof_begin(LOOMHIP_KT_DOWN, st);
             ok = launch_dmmv(L.down_t, nt, false, dn, st);
-            prof_end(ph, st);
+            prof_end(ph, st, ok);
             if (!ok)
                 return tables_done(fail(LOOMHIP_ERR_ARG, "moe_cached: down partials exceed LDS"));
         }

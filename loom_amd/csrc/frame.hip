@@ -1140,7 +1140,7 @@ static bool frame_matvec(int t, const void *wt, int rows, int cols, const FrameW
     p.rpw = mq ? 0 : dmmv_pick_rpw(t, cols, rows, w.n_groups, w.nt, false);
     const int ph = prof_begin(tag, st);
     const bool ok = mq ? launch_mmq(t, n > 16 ? mmq_group : 16, false, p, st) : launch_dmmv(t, w.nt, false, p, st);
-    prof_end(ph, st);
+    prof_end(ph, st, ok);
     return ok;
 }
 
@@ -1161,7 +1161,7 @@ static bool frame_self(int t, const void *wt, const void *w2, int rows, int cols
     sp.n_seg = 1;
     const int ph = prof_begin(tag, st);
     const bool ok = launch_dmmv_self(w2 != nullptr, sp, x, cols, norm_w, eps, st);
-    prof_end(ph, st);
+    prof_end(ph, st, ok);
     return ok;
 }
 
@@ -1195,7 +1195,7 @@ static bool frame_qkv(const loomhip_layer &l, const FrameDims &D, const FrameWs 
             return false;
         const int ph = prof_begin(LOOMHIP_KT_QKV, st);
         *fused = launch_dmmv_self(false, sp, w.x, 0, l.attn_norm, D.eps, st);
-        prof_end(ph, st);
+        prof_end(ph, st, *fused);
         return *fused;
     }
     // from QKV_MMQ_MIN lanes: the matrix cores, the three matrices in one
@@ -1205,13 +1205,13 @@ static bool frame_qkv(const loomhip_layer &l, const FrameDims &D, const FrameWs 
         mp.base.ident_n = (int)n;
         const int ph = prof_begin(LOOMHIP_KT_QKV, st);
         const bool ok = launch_mmq_seg(mp, st);
-        prof_end(ph, st);
+        prof_end(ph, st, ok);
         if (ok)
             return true;
     }
     const int ph = prof_begin(LOOMHIP_KT_QKV, st);
     const bool ok = launch_dmmv_seg(w.nt, sp, st);
-    prof_end(ph, st);
+    prof_end(ph, st, ok);
     return ok;
 }
 

@@ -70,8 +70,10 @@ bool launch_dmmv_self(bool fused, DmmvSegParams sp, const float *x, int x_stride
 
 void note_launch();
 // Event timing around tagged launches (LOOMHIP_KT_*); -1 when disabled.
+// launched false: nothing ran between the two (a declined launch), no record
+// is kept.
 int prof_begin(int tag, hipStream_t st);
-void prof_end(int handle, hipStream_t st);
+void prof_end(int handle, hipStream_t st, bool launched = true);
 
 void launch_quant_act(int wtype, const float *x, int cols, int x_stride, int nvec, QAct qa,
                       hipStream_t st);

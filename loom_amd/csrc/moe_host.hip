@@ -352,7 +352,7 @@ static int moe_run(const MoeRun &m, const float *normed, const float *logits_in,
     gu.rpw = mq ? 0 : dmmv_pick_rpw(m.gate_t, (int)m.dim, (int)m.ffn, exp_groups, nt, true);
     int ph = prof_begin(LOOMHIP_KT_GATE_UP, st);
     bool launched = mq ? launch_mmq(m.gate_t, nt, true, gu, st) : launch_dmmv(m.gate_t, nt, true, gu, st);
-    prof_end(ph, st);
+    prof_end(ph, st, launched);
     if (!launched)
         return fail(LOOMHIP_ERR_ARG, "moe: gate/up partials exceed LDS");
 
@@ -377,7 +377,7 @@ static int moe_run(const MoeRun &m, const float *normed, const float *logits_in,
     dn.rpw = mq ? 0 : dmmv_pick_rpw(m.down_t, (int)m.ffn, (int)m.dim, exp_groups, nt, false);
     ph = prof_begin(LOOMHIP_KT_DOWN, st);
     launched = mq ? launch_mmq(m.down_t, nt, false, dn, st) : launch_dmmv(m.down_t, nt, false, dn, st);
-    prof_end(ph, st);
+    prof_end(ph, st, launched);
     if (!launched)
         return fail(LOOMHIP_ERR_ARG, "moe: down partials exceed LDS");
 

@@ -56,9 +56,15 @@ int prof_begin(int tag, hipStream_t st) {
     return (int)g_prof_recs.size() - 1;
 }
 
-void prof_end(int handle, hipStream_t st) {
+void prof_end(int handle, hipStream_t st, bool launched) {
     if (handle < 0 || handle >= (int)g_prof_recs.size())
         return;
+    if (!launched) { // the newest record: every begin is ended before the next
+        g_prof_pool.push_back(g_prof_recs[handle].a);
+        g_prof_pool.push_back(g_prof_recs[handle].b);
+        g_prof_recs.erase(g_prof_recs.begin() + handle);
+        return;
+    }
     (void)hipEventRecord(g_prof_recs[handle].b, st);
 }
 
@@ -240,7 +246,7 @@ int matvec_dev_impl(int t, float *out, const void *w, const float *x, size_t n, 
         sp.n_seg = 1;
         const int ph = prof_begin(LOOMHIP_KT_DENSE, st);
         const bool done = launch_dmmv_self(false, sp, x, (int)cols, nullptr, 0.0f, st);
-        prof_end(ph, st);
+        prof_end(ph, st, done);
         if (done)
             return LOOMHIP_OK;
     }
@@ -278,7 +284,7 @@ int matvec_dev_impl(int t, float *out, const void *w, const float *x, size_t n, 
     p.ident_n = mq ? (int)n : 0;
     const int ph = prof_begin(LOOMHIP_KT_DENSE, st);
     const bool launched = mq ? launch_mmq(t, nt, false, p, st) : launch_dmmv(t, nt, false, p, st);
-    prof_end(ph, st);
+    prof_end(ph, st, launched);
     if (!launched)
         return fail(LOOMHIP_DECLINED, "dmmv: partials exceed LDS for %zu columns", cols);
     return LOOMHIP_OK;

@@ -60,3 +60,55 @@ def test_one_vector_matvec_dev_over_its_input(oracle, t, rows, cols, place):
     torch.cuda.synchronize()
     want = oracle.matvec(t, raw, x, rows, cols)
     assert np.array_equal(out.cpu().numpy().view(np.uint32), want.view(np.uint32))
+
+
+@pytest.mark.parametrize("t,rows,cols,n", [(Q4_0, 768, 2048, 1), (Q4_K, 4096, 4096, 1), (Q8_0, 4097, 2048, 1),
+                                           (Q8_0, 64, 2080, 1), (Q4_K, 768, 2048, 3), (Q6_K, 300, 2048, 9)])
+def test_one_timing_record_per_matvec(oracle, t, rows, cols, n):
+    """A call that declines the one-launch form (wider rows, more work groups)
+    before it runs the two adds one sample to the matvec's timing, not two."""
+    import torch
+
+    import loom_amd
+    from loom_amd import backend as be
+
+    loom_amd.init(0)
+    w = torch.zeros(loom_amd.plane_bytes(t, rows, cols), dtype=torch.uint8, device="cuda")
+    x, out = torch.zeros(n, cols, device="cuda"), torch.empty(n, rows, device="cuda")
+    be.profileKernels(True)
+    try:
+        for _ in range(3):
+            assert be.matvec_dev(t, out, w, x, n, rows, cols) == loom_amd.OK
+        torch.cuda.synchronize()
+        assert be.kernelStats()["dense"]["count"] == 3
+    finally:
+        be.profileKernels(False)
+
+
+@pytest.mark.parametrize("n", [1, 6])
+def test_one_timing_record_per_frame_stage(n):
+    """The same inside the frame: q, k and v in Q8_0 decline the matrix-core
+    launch at 6 lanes; at one lane wo and the dense down decline the one-launch
+    matvec where their rows are wider than 2048."""
+    import dataclasses
+
+    import torch
+
+    import loom_amd
+    from loom_amd import backend as be
+    from loom_amd import frame as lh
+
+    loom_amd.init(0)
+    layers = 3
+    spec = dataclasses.replace(lh.stories15m(ctx_len=32), dim=512, n_layers=layers, vocab=512, n_heads=40,
+                               n_kv_heads=8, head_dim=64, rope_dim=64, ffn=2080, embed_t=Q8_0, output_t=Q8_0,
+                               wq_t=Q8_0, wk_t=Q8_0, wv_t=Q8_0, wo_t=Q8_0, ffn_gate_t=Q8_0, ffn_down_t=Q8_0)
+    dec = lh.Decoder(lh.DeviceModel.synth(spec, seed=3), n)
+    be.profileKernels(True)
+    try:
+        assert dec.step() == loom_amd.OK
+        torch.cuda.synchronize()
+        st = be.kernelStats()
+        assert [st[k]["count"] for k in ("qkv", "wo", "dense")] == [layers] * 3
+    finally:
+        be.profileKernels(False)
