@@ -1720,10 +1720,15 @@ static bool mmq_oneshot(int t, int cols, int max_tok, bool fused) {
     return mmq_shape(16, cols, (max_tok + 15) / 16, fused, rg, ks, sbw);
 }
 
-// The streamed kernels' shapes: whole blocks, byte offsets in 32 bits.
+// The streamed kernels' shapes: whole blocks, the K-quants' block scales of 16
+// tokens in the CU's LDS (Q4_K to 532480 columns, Q6_K to 531456; groups of 32
+// end at 4096, the 32-value blocks hold one unit's), byte offsets in 32 bits.
+constexpr size_t MMW_LDS_MAX = 160 * 1024;
 static bool mmw_shape(int t, int rows, int cols, bool fused) {
     if ((t != LH_Q4_K && t != LH_Q6_K && t != LH_Q8_0 && t != LH_Q4_0) || cols < block_elems(t) ||
         cols % block_elems(t) || (fused && t == LH_Q6_K))
+        return false;
+    if (is_k(t) && (t == LH_Q4_K ? mmw_lds<LH_Q4_K, 1, false>(cols) : mmw_lds<LH_Q6_K, 1, false>(cols)) > MMW_LDS_MAX)
         return false;
     return (size_t)rows * (cols / block_elems(t)) * block_bytes(t) < ((size_t)1 << 32);
 }

@@ -153,3 +153,28 @@ def test_moe_layer_streamed_experts(be, oracle, t, dim, ffn, n):
     torch.cuda.synchronize()
     assert np.array_equal(ids.cpu().numpy().astype(np.uint32), wid)
     assert np.array_equal(out.cpu().numpy().view(np.uint32), want.view(np.uint32))
+
+
+# the widest rows whose block scales fit the LDS, and one block more, which no kernel serves
+@pytest.mark.parametrize("t,cols,served", [(Q6_K, 2076 * 256, True), (Q6_K, 2077 * 256, False), (Q4_K, 2080 * 256, True),
+                                           (Q4_K, 2081 * 256, False)])
+def test_widest_streamed_rows(be, oracle, t, cols, served):
+    import torch
+
+    import loom_amd
+
+    rows, n = 512, 256
+    rng = np.random.default_rng(cols)
+    raw = npref.pinned_scale_blocks(t, rows, cols, rng)
+    w = be.repack_dev(t, torch.from_numpy(raw).cuda(), rows, cols, 1)
+    x = torch.randn(n, cols, generator=torch.Generator(device="cuda").manual_seed(t), device="cuda")
+    out = torch.full((n, rows), 7.0, device="cuda")
+    rc = be.matvec_dev(t, out, w, x, n, rows, cols)
+    torch.cuda.synchronize()
+    if not served:
+        assert rc == loom_amd.DECLINED and bool((out == 7.0).all())
+        return
+    assert rc == loom_amd.OK
+    for k in (0, 100, n - 1):
+        want = oracle.matvec(t, raw, x[k].cpu().numpy(), rows, cols)
+        assert np.array_equal(out[k].cpu().numpy().view(np.uint32), want.view(np.uint32)), k
