@@ -1744,10 +1744,20 @@ static long lane_pairs(int rows, int n) { return (long)((rows + 15) / 16) * ((n 
 // 13.1 / 9.8; Q6_K 16384 x 4096 at 16 (1024) 32.7 / 20.6; fused 2048 x 7168 at
 // 24 (256) 25.6 / 32.1, at 64 (512) 44.8 / 32.6; fused 4096 x 2048 at 24 (512)
 // 12.7 / 13.2, at 64 (1024) 20.4 / 14.0.
+// The 32-value blocks' one-shot kernel fills a CU's LDS, so it takes one round
+// of the chip per 256 pairs; rows of up to 1536 columns stream as fast as two
+// rounds, of 2048 as three.  us per call, dot4 / one-shot / streamed: Q4_0 4096
+// x 1024 at 24 (512 pairs) 14.1 / 14.5 / 10.1, 2500 x 1536 at 32 (314) 14.2 /
+// 15.3 / 12.3, 2500 x 1984 at 32 13.8 / 11.8 / 14.4, at 63 (628) 22.1 / 15.8 /
+// 14.6, 4096 x 4096 at 24 (512) 32.3 / 17.6 / 26.1.
 constexpr long MMW_MIN_WAVES = 768, MMW_MIN_WAVES_FUSED = 512;
 static bool lanes_streamed(int t, int rows, int cols, int n, bool fused) {
-    return mmw_shape(t, rows, cols, fused) &&
-           lane_pairs(rows, n) >= (fused ? MMW_MIN_WAVES_FUSED : MMW_MIN_WAVES);
+    const long pairs = lane_pairs(rows, n);
+    if (!mmw_shape(t, rows, cols, fused))
+        return false;
+    if (!is_k(t) && !fused && ((cols <= 1536 && pairs > 256) || (cols <= MMW_XL_COLS && pairs > 512)))
+        return true;
+    return pairs >= (fused ? MMW_MIN_WAVES_FUSED : MMW_MIN_WAVES);
 }
 
 // Expert groups of K-quants with fewer (group, row tile, matrix) streams than
@@ -1777,28 +1787,74 @@ static bool lanes_tiled(int t, int rows, int cols, int n) {
     return t == LH_Q4_K ? lane_pairs(rows, n) * 5 >= room * 4 : lane_pairs(rows, n) * 3 >= room * 2;
 }
 
+// Q8_0 / Q4_0: whether the matrix cores take n vectors against one matrix from
+// the dot4 matvec.  us per call (quantization and matmul, back to back in a
+// graph, weights from a ring past the caches), dot4 / matrix cores.
+// One-shot shapes (whole 64-value spans, 512 to 4096 columns): the kernel costs
+// about the same for any matrix of one round, a little less where a row's
+// bytes are no multiple of the 128-byte line; the dot4 matvec's time grows
+// with the row length, and with n * rows * cols once the chip is full.
+//   8 vectors and up, over 2048 columns, or over 1024 for Q8_0 or rows off the
+//     line: 300 x 3072 at 8 Q4_0 11.6 / 9.2, Q8_0 12.4 / 9.3; 200 x 4096 at 16
+//     12.6 / 10.5 and 15.8 / 10.6; Q8_0 300 x 1088 at 8 7.9 / 6.9, 300 x 1536
+//     8.6 / 8.4; Q4_0 300 x 1088 7.2 / 6.9, 300 x 1984 7.4 / 7.0.
+//   Narrower, from n * rows * cols of 40 Mi, off the line 20 Mi: 768 x 1024 at
+//     32 (24 Mi) Q8_0 8.2 / 9.1, at 63 (47) 9.4 / 9.2; Q4_0 1000 x 1536 at 16
+//     (23) 8.0 / 9.1, at 63 (92) 12.8 / 9.7; 2048 x 512 at 8 (8) 6.6 / 8.4;
+//     1000 x 960 at 16 (15) 6.8 / 7.2, at 32 (29) 7.7 / 7.2.
+//   From 5 vectors at 8 Mi weights: Q4_0 4096 x 2048 9.2 / 8.9, 4096 x 4096
+//     13.4 / 10.0; 2048 x 2048 7.9 / 8.8.
+// Shapes only the streamed kernel serves: up to 2048 columns (the vectors' rows
+// staged whole) its time grows with the columns alone until the chip is
+// full, the dot4 matvec's with n * rows too.
+//   Under 256 columns from 8 vectors (512 x 160 Q4_0 7.0 / 5.6, Q8_0 5.8 / 5.5);
+//   under 512 from n * rows of 32 Ki (Q4_0 4096 x 288 at 8 6.7 / 6.1, Q8_0 1500 x
+//     288 at 16 5.8 / 6.6, 3000 x 416 at 16 7.3 / 7.3);
+//   to 2048 from 40000 + 12 * cols (6000 x 864 at 8 (48000) Q4_0 8.7 / 8.2, Q8_0
+//     8.4 / 8.4; 1500 x 2016 at 16 (24000) 9.1 / 14.4 and 10.3 / 14.3, 6000 x
+//     2016 at 12 (72000) 15.1 / 14.5 and 16.2 / 14.6);
+//   wider from 512 pairs (Q8_0 4096 x 11008 at 16 vectors, 256 pairs, 60.5 /
+//     56.5, Q4_0 47.9 / 58.2; at 32, 512 pairs, 111 / 57 and 84 / 59).
+static bool lanes32_on_cores(int t, int rows, int cols, int n) {
+    const size_t size = (size_t)rows * cols;
+    if (mmq32_supported(t, cols, 16, false)) {
+        if (n < 8)
+            return n >= 5 && size >= ((size_t)8 << 20);
+        const bool line = cols / 32 * (t == LH_Q8_0 ? 32 : 16) % 128 == 0;
+        if (cols > 2048 || (cols > 1024 && (t == LH_Q8_0 || !line)))
+            return true;
+        return n * size >= ((size_t)(line ? 40 : 20) << 20);
+    }
+    if (!mmw_shape(t, rows, cols, false))
+        return false;
+    if (cols > MMW_XL_COLS)
+        return n >= (size >= ((size_t)8 << 20) ? 5 : 8) && lane_pairs(rows, n) >= 512;
+    if (cols < 256)
+        return n >= 8;
+    return n >= 5 && (long)n * rows >= (cols < 512 ? 32768 : 40000 + 12 * cols);
+}
+
 // n vectors against one [rows][cols] matrix (or a fused pair): whether the
-// matrix cores take them from the dot4 matvec.  By type and size, us per
-// launch, dot4 / matrix cores: Q4_K 4096 x 4096 at 5 vectors 11.4 / 9.1,
-// 1024 x 2048 6.7 / 6.6; Q6_K at 5 10.8 / 10.4 and 6.6 / 7.1, at 8 12.5 /
-// 10.6 and 7.8 / 7.2; Q8_0 at 5 15.2 / 10.0 and 7.8 / 8.5, at 8 19.7 / 10.5
-// and 9.8 / 8.8 (Q4_0 8.9 / 8.7); 768 x 288 at 32 6.2 / 7.4.  A shape only the
-// streamed kernels serve needs their rows staged whole or 512 pairs (Q8_0
-// 4096 x 11008 at 16 vectors, 256 pairs, 60.5 / 56.5, Q4_0 47.9 / 58.2; at
-// 32, 512 pairs, 111 / 57 and 84 / 59).  A fused pair: from 16 as measured
-// for Q4_K (2048 x 7168 at 8 vectors 16 / 24, at 24 47 / 25).
+// matrix cores take them from the dot4 matvec.  By type, us per launch, dot4 /
+// matrix cores: Q4_K 4096 x 4096 at 5 vectors 11.4 / 9.1, 1024 x 2048 6.7 /
+// 6.6; Q6_K at 5 10.8 / 10.4 and 6.6 / 7.1, at 8 12.5 / 10.6 and 7.8 / 7.2; one
+// Q8_0 / Q4_0 matrix lanes32_on_cores.  A shape only the streamed kernels
+// serve needs 512 pairs.  A fused pair: Q4_K from 16 (2048 x 7168 at 8 vectors
+// 16 / 24, at 24 47 / 25); Q8_0 / Q4_0, streamed only, us per call: 4096 x 2048
+// at 16 (256 pairs) 29.2 / 23.9 and 24.7 / 23.7, at 24 (512) 37.1 / 23.8 and
+// 33.4 / 23.7; 2048 x 2048 at 32 (256) 27.5 / 22.8 and 24.6 / 23.7, at 64 (512)
+// 44.2 / 23.0 and 42.2 / 23.9; 11008 x 4096 at 5 (688) 57.8 / 32.2 and 50.3 /
+// 32.8; 2048 x 7168 at 32 (256) 104 / 69 and 85 / 70.
 bool mmq_dense(int t, int rows, int cols, int n, bool fused) {
     if (rows < 1 || n < 1)
         return false;
-    const int min_k = fused ? 16 : t == LH_Q4_K ? 5 : 8;
+    if (!is_k(t) && !fused)
+        return lanes32_on_cores(t, rows, cols, n);
     const size_t size = (size_t)rows * cols;
     const int min_32 = size >= ((size_t)8 << 20) ? 5 : size >= ((size_t)1 << 20) ? 8 : 64;
-    if (n < (is_k(t) ? min_k : min_32))
+    if (n < (!is_k(t) ? min_32 : fused ? 16 : t == LH_Q4_K ? 5 : 8))
         return false;
-    if (mmq_oneshot(t, cols, 16, fused))
-        return true;
-    return mmw_shape(t, rows, cols, fused) &&
-           (lane_pairs(rows, n) >= 512 || (!is_k(t) && !fused && cols <= MMW_XL_COLS));
+    return mmq_oneshot(t, cols, 16, fused) || (mmw_shape(t, rows, cols, fused) && lane_pairs(rows, n) >= 512);
 }
 
 // The expert matmuls of n tokens: whether they run on the matrix cores in

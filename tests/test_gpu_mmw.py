@@ -121,6 +121,20 @@ def test_streamed_32_block_matmul_edges(be, oracle, t, rows, cols, n):
     _check(be, oracle, t, raw, xs, rows, cols)
 
 
+# either side of each line by which a Q8_0 / Q4_0 matmul is routed: rows on and off the 128-byte line (multiples
+# of 128 columns in Q8_0, 256 in Q4_0), widths of 1024, 1536 and 2048, one round of one-shot work groups and two
+@pytest.mark.parametrize("t", [Q4_0, Q8_0])
+@pytest.mark.parametrize("rows,cols,n", [(200, 4096, 16), (300, 3072, 7), (300, 3072, 8), (257, 1088, 8), (300, 1280, 9),
+                                         (768, 1024, 48), (768, 1024, 63), (1000, 960, 24), (2048, 512, 8),
+                                         (8192, 512, 12), (2500, 1536, 32), (2500, 1984, 32), (2500, 1984, 47),
+                                         (1500, 2016, 16), (6000, 2016, 12), (4096, 288, 8), (512, 160, 8), (512, 256, 9)])
+def test_32_block_routes(be, oracle, t, rows, cols, n):
+    rng = np.random.default_rng(rows + cols + n + t)
+    raw = npref.pinned_scale_blocks(t, rows, cols, rng)
+    xs = np.stack([oracle.normal(cols, 100 * n + k, 0.0, float(k % 5 + 1)) for k in range(n)])
+    _check(be, oracle, t, raw, xs, rows, cols)
+
+
 # five to fifteen vectors on the matrix cores (one-shot), rows too wide for 32 lanes a wave
 @pytest.mark.parametrize("t,rows,cols,n", [(Q4_K, 300, 2048, 5), (Q4_K, 77, 8192, 17), (Q6_K, 300, 768, 8),
                                            (Q6_K, 130, 8192, 9), (Q8_0, 2100, 4096, 5), (Q4_0, 1100, 1024, 11),
