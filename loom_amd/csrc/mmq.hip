@@ -1834,12 +1834,33 @@ static bool lanes32_on_cores(int t, int rows, int cols, int n) {
     return n >= 5 && (long)n * rows >= (cols < 512 ? 32768 : 40000 + 12 * cols);
 }
 
+// The same for one K-quant matrix.  Q4_K from 5 vectors, Q6_K from 8 (us per
+// launch, dot4 / matrix cores: Q4_K 4096 x 4096 at 5 vectors 11.4 / 9.1, 1024 x
+// 2048 6.7 / 6.6; Q6_K at 5 10.8 / 10.4 and 6.6 / 7.1, at 8 12.5 / 10.6 and 7.8 /
+// 7.2), but below 16 vectors (us per call)
+//   Q6_K rows of one or two blocks (most of the one-shot kernel's waves idle) from
+//     n * rows * cols of 14 Mi: 1004 x 512 at 11 6.5 / 6.9, 2500 x 512 at 12 7.3 /
+//     6.9, 8192 x 512 at 8 7.8 / 7.3;
+//   rows of 20 to 24 blocks, whose waves hold four blocks for three, from 2048
+//     rows: Q6_K 900 x 4864 at 9 13.4 / 12.7, 300 x 5120 12.5 / 13.3, 1900 x 6144
+//     14.5 / 15.1, 2500 x 6144 at 8 15.9 / 14.9; Q4_K only where the row's bytes are a multiple of
+//     the 128-byte line and under 8 vectors: 1000 x 6144 at 5 11.1 / 12.6, at 8
+//     14.6 / 13.2, 1000 x 5632 at 5 11.1 / 11.0.
+static bool lanes_k_on_cores(int t, int rows, int cols, int n) {
+    const int nb = cols / 256;
+    if (n < (t == LH_Q4_K ? 5 : 8))
+        return false;
+    if (n < 16 && t == LH_Q6_K && nb <= 2 && (size_t)n * rows * cols < ((size_t)14 << 20))
+        return false;
+    if (n < 16 && nb >= 20 && nb <= 24 && rows < 2048 && (t == LH_Q6_K || (n < 8 && nb * 144 % 128 == 0)))
+        return false;
+    return mmq_oneshot(t, cols, 16, false) || (mmw_shape(t, rows, cols, false) && lane_pairs(rows, n) >= 512);
+}
+
 // n vectors against one [rows][cols] matrix (or a fused pair): whether the
-// matrix cores take them from the dot4 matvec.  By type, us per launch, dot4 /
-// matrix cores: Q4_K 4096 x 4096 at 5 vectors 11.4 / 9.1, 1024 x 2048 6.7 /
-// 6.6; Q6_K at 5 10.8 / 10.4 and 6.6 / 7.1, at 8 12.5 / 10.6 and 7.8 / 7.2; one
-// Q8_0 / Q4_0 matrix lanes32_on_cores.  A shape only the streamed kernels
-// serve needs 512 pairs.  A fused pair: Q4_K from 16 (2048 x 7168 at 8 vectors
+// matrix cores take them from the dot4 matvec.  One matrix: lanes32_on_cores,
+// lanes_k_on_cores.  A shape only the streamed kernels serve needs 512 pairs.  A
+// fused pair, us per launch, dot4 / matrix cores: Q4_K from 16 (2048 x 7168 at 8 vectors
 // 16 / 24, at 24 47 / 25); Q8_0 / Q4_0, streamed only, us per call: 4096 x 2048
 // at 16 (256 pairs) 29.2 / 23.9 and 24.7 / 23.7, at 24 (512) 37.1 / 23.8 and
 // 33.4 / 23.7; 2048 x 2048 at 32 (256) 27.5 / 22.8 and 24.6 / 23.7, at 64 (512)
@@ -1848,13 +1869,14 @@ static bool lanes32_on_cores(int t, int rows, int cols, int n) {
 bool mmq_dense(int t, int rows, int cols, int n, bool fused) {
     if (rows < 1 || n < 1)
         return false;
-    if (!is_k(t) && !fused)
-        return lanes32_on_cores(t, rows, cols, n);
-    const size_t size = (size_t)rows * cols;
-    const int min_32 = size >= ((size_t)8 << 20) ? 5 : size >= ((size_t)1 << 20) ? 8 : 64;
-    if (n < (!is_k(t) ? min_32 : fused ? 16 : t == LH_Q4_K ? 5 : 8))
+    if (t != LH_Q4_0 && t != LH_Q8_0 && !is_k(t))
         return false;
-    return mmq_oneshot(t, cols, 16, fused) || (mmw_shape(t, rows, cols, fused) && lane_pairs(rows, n) >= 512);
+    if (!fused)
+        return is_k(t) ? lanes_k_on_cores(t, rows, cols, n) : lanes32_on_cores(t, rows, cols, n);
+    const size_t size = (size_t)rows * cols;
+    if (n < (is_k(t) ? 16 : size >= ((size_t)8 << 20) ? 5 : size >= ((size_t)1 << 20) ? 8 : 64))
+        return false;
+    return mmq_oneshot(t, cols, 16, true) || (mmw_shape(t, rows, cols, true) && lane_pairs(rows, n) >= 512);
 }
 
 // The expert matmuls of n tokens: whether they run on the matrix cores in

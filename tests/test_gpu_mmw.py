@@ -135,6 +135,17 @@ def test_32_block_routes(be, oracle, t, rows, cols, n):
     _check(be, oracle, t, raw, xs, rows, cols)
 
 
+# the same for the K-quants under 16 vectors: rows of one and two blocks, rows of 20 to 24 around 2048 rows
+@pytest.mark.parametrize("t,rows,cols,n", [(Q6_K, 1004, 512, 11), (Q6_K, 2500, 512, 12), (Q6_K, 7168, 256, 8),
+                                           (Q6_K, 2047, 5120, 8), (Q6_K, 300, 4864, 8), (Q6_K, 2048, 6144, 8), (Q6_K, 300, 5120, 16),
+                                           (Q4_K, 1000, 6144, 7), (Q4_K, 1000, 6144, 8), (Q4_K, 300, 5632, 5)])
+def test_k_quant_routes(be, oracle, t, rows, cols, n):
+    rng = np.random.default_rng(rows + cols + n + t)
+    raw = npref.pinned_scale_blocks(t, rows, cols, rng)
+    xs = np.stack([oracle.normal(cols, 100 * n + k, 0.0, float(k % 5 + 1)) for k in range(n)])
+    _check(be, oracle, t, raw, xs, rows, cols)
+
+
 # five to fifteen vectors on the matrix cores (one-shot), rows too wide for 32 lanes a wave
 @pytest.mark.parametrize("t,rows,cols,n", [(Q4_K, 300, 2048, 5), (Q4_K, 77, 8192, 17), (Q6_K, 300, 768, 8),
                                            (Q6_K, 130, 8192, 9), (Q8_0, 2100, 4096, 5), (Q4_0, 1100, 1024, 11),
