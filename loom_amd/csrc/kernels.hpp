@@ -92,11 +92,11 @@ bool dmmv_supported(int t, int cols);
 bool launch_dmmv(int t, int nt, bool fused, const DmmvParams &p, hipStream_t st);
 // Matrix-core variant, the same results bit for bit.  mmq_dense: whether it
 // takes n vectors against one matrix (a fused pair) from the dot4 matvec;
-// mmq_experts: whether it takes the expert matmuls of n tokens, in groups of
-// up to 16.  launch_mmq: groups of up to max_tok (<= 32) tokens; false
+// mmq_experts: whether it takes the expert matmuls of n tokens (top-k of E
+// experts), in groups of up to 16.  launch_mmq: groups of up to max_tok (<= 32) tokens; false
 // (nothing launched) for a type or shape it does not serve.
 bool mmq_dense(int t, int rows, int cols, int n, bool fused);
-bool mmq_experts(int gate_t, int down_t, int dim, int ffn, int n);
+bool mmq_experts(int gate_t, int down_t, int dim, int ffn, int n, int k, int E);
 bool launch_mmq(int t, int max_tok, bool fused, const DmmvParams &p, hipStream_t st);
 bool launch_mmq_seg(DmmvSegParams sp, hipStream_t st);
 // Rows per wave chosen for a launch of `rows` rows x `groups` groups.

@@ -1879,22 +1879,39 @@ bool mmq_dense(int t, int rows, int cols, int n, bool fused) {
     return mmq_oneshot(t, cols, 16, true) || (mmw_shape(t, rows, cols, true) && lane_pairs(rows, n) >= 512);
 }
 
-// The expert matmuls of n tokens: whether they run on the matrix cores in
-// groups of 16.  By type and expert size, us per layer with the dot4 / matrix
-// core matmuls, Zipf-skewed router: Q4_K + Q6_K 2048 x 768 x 128 at 5 tokens
-// 48.8 / 46.4 (uniform 58.3 / 56.8), 1024 x 512 x 32 at 10 35.2 / 32.1; Q8_0
-// 2048 x 768 at 8 66.7 / 61.7 (uniform 79.3 / 86.7), at 12 90.5 / 66.2 (113 /
-// 97), Q4_0 at 12 76.3 / 57.5; 7168 x 2048 x 16 at 5 Q8_0 183 / 150, Q4_0 142 /
-// 116; Q8_0 1024 x 512 x 32 at 15 35.2 / 40.1.
-static int experts_min(int t, size_t size) {
+// The expert matmuls of n tokens, pairs of them with E experts: whether they run
+// on the matrix cores in groups of 16.  By type and expert size, us per layer
+// with the dot4 / matrix core matmuls, Zipf-skewed router (uniform):
+//   K-quants from 5 tokens at 1.5 M weights, else 10: 2048 x 768 x 128 top-8 at
+//     5 47.9 / 44.5 (53.8 / 54.5), 1536 x 768 x 64 top-6 at 10 50.3 / 43.3, 1024
+//     x 512 x 32 top-4 at 10 33.8 / 31.2;
+//   Q8_0 / Q4_0 from 5 at 8 M (4096 x 2048 x 16 top-4 108 / 72 and 87 / 68), 12
+//     at 1.5 M (1536 x 1280 x 60 top-6 80 / 62 and 67 / 57, uniform 111 / 89 and
+//     79 / 64; 2048 x 768 x 128 89 / 69 and 74 / 61; Q4_0 at 8 54.5 / 53.1,
+//     uniform 62 / 69), else 20 (1024 x 768 x 64 top-6 55.3 / 48.9 and 54.3 / 46.6),
+//     of under 750000 weights with 100 pairs or more than three pairs per
+//     expert (there the dot4 form goes to groups of eight): 1024 x 512 x 32 top-4
+//     at 20 37.3 / 41.5 and 38.0 / 40.4, at 24 40.5 / 41.5 and 41.2 / 40.7, at 26 (768 x
+//     384) 38.1 / 37.5 and 39.4 / 36.9; x 64 top-8 at 20 52.5 / 49.5 and 53.1 / 47.1; x
+//     16 top-4 at 20 44.3 / 41.0 and 42.7 / 39.7.
+// Inputs of over 2048 columns (not staged whole) also need row tiles to stream:
+// 4096 x 768 x 64 top-4 K-quants at 5 (960 (pair, tile) streams) 44.4 / 49.3, at 7
+// (1344) 49.1 / 49.9, with a Q4_K down 48.6 / 45.5; 4096 x 1024 x 32 top-4 at 5 (1280) 45.7 / 49.6, at 7 (1792)
+// 55.3 / 53.7; 4096 x 1280 x 32 at 5 (1600) 58.2 / 54.0.
+constexpr long EXPERT_MIN_STREAMS = 1300;
+static bool experts_take(int t, size_t size, int n, int pairs, int E) {
     if (is_k(t))
-        return size >= 1500000 ? 5 : 10;
-    return size >= 8000000 ? 5 : size >= 1500000 ? 12 : 20;
+        return n >= (size >= 1500000 ? 5 : 10);
+    if (size >= 1500000)
+        return n >= (size >= 8000000 ? 5 : 12);
+    return n >= 20 && (size >= 750000 || pairs >= 100 || pairs > 3 * E);
 }
-bool mmq_experts(int gate_t, int down_t, int dim, int ffn, int n) {
+bool mmq_experts(int gate_t, int down_t, int dim, int ffn, int n, int k, int E) {
     const size_t size = (size_t)dim * ffn;
-    return mmw_shape(gate_t, ffn, dim, true) && mmw_shape(down_t, dim, ffn, false) && n >= experts_min(gate_t, size) &&
-           n >= experts_min(down_t, size);
+    if (!mmw_shape(gate_t, ffn, dim, true) || !mmw_shape(down_t, dim, ffn, false) ||
+        (dim > MMW_XL_COLS && (long)n * k * ((ffn + 15) / 16) < EXPERT_MIN_STREAMS))
+        return false;
+    return experts_take(gate_t, size, n, n * k, E) && experts_take(down_t, size, n, n * k, E);
 }
 
 template <int T, int MT, bool FUSED>

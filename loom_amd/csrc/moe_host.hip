@@ -207,7 +207,7 @@ static int moe_run(const MoeRun &m, const float *normed, const float *logits_in,
     const bool decode = n <= DECODE_MAX_TOK && decode_supported(m.gate_t, m.down_t, (int)m.ffn);
     // matrix cores for the expert matmuls where mmq_experts takes them, groups
     // of up to 16 tokens per expert
-    const bool mq = !decode && mmq_experts(m.gate_t, m.down_t, (int)m.dim, (int)m.ffn, (int)n);
+    const bool mq = !decode && mmq_experts(m.gate_t, m.down_t, (int)m.dim, (int)m.ffn, (int)n, (int)m.k, (int)m.E);
     const int nt = mq ? 16 : moe_nt(n, m.k, m.E);
     const int maxg = moe_max_groups((int)n, (int)m.k, (int)m.E, nt);
     // workspace layout

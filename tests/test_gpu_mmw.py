@@ -159,15 +159,26 @@ def test_matmul_from_five_vectors(be, oracle, t, rows, cols, n):
 
 @pytest.mark.parametrize("t,dim,ffn,n", [(Q8_0, 288, 96, 21), (Q4_0, 544, 288, 40), (Q8_0, 2080, 768, 12),
                                          (Q4_0, 1024, 1536, 13), (Q4_K, 512, 256, 10), (Q4_K, 2304, 768, 5),
-                                         (Q4_K, 2304, 3072, 17), (Q4_K, 4352, 1536, 17)])
+                                         (Q4_K, 2304, 3072, 17), (Q4_K, 4352, 1536, 17), (Q4_K, 2304, 768, 9), (Q4_K, 2304, 768, 10)])
 def test_moe_layer_streamed_experts(be, oracle, t, dim, ffn, n):
     """The routed layer with its expert matmuls in groups of 16 for every type
     (streamed; Q4_K gate/up streamed from 2304 x 3072 on, down from 4352 x
-    1536, one-shot below): ids, gates and output bits against lo_moe_batch_union."""
+    1536, one-shot below; 2304 x 768 from 10 tokens, the dot4 matvec before):
+    ids, gates and output bits against lo_moe_batch_union."""
+    _moe_layer(be, oracle, t, dim, ffn, 6, 3, n)
+
+
+# small Q8_0 / Q4_0 experts: 20 tokens and either 100 pairs or more than three per expert
+@pytest.mark.parametrize("t", [Q4_0, Q8_0])
+@pytest.mark.parametrize("E,k,n", [(32, 4, 24), (32, 4, 25), (16, 4, 19), (16, 4, 20)])
+def test_moe_layer_small_experts(be, oracle, t, E, k, n):
+    _moe_layer(be, oracle, t, 768, 384, E, k, n)
+
+
+def _moe_layer(be, oracle, t, dim, ffn, E, k, n):
     import torch
     from test_gpu_moe import _dev_layer, make_layer
 
-    E, k = 6, 3
     w = make_layer(oracle, dim, ffn, E, k, seed=dim + n, gate_t=t, down_t=t)
     layer = _dev_layer(be, w)
     xs = np.stack([oracle.normal(dim, 700 + i, 0.0, 1.0) for i in range(n)])
