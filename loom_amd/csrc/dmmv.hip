@@ -285,7 +285,11 @@ __global__ __launch_bounds__(256, 4) void dmmv_self_kernel(DmmvSegParams sp, con
 // more than the launch it saves.  Measured, us back to back, two launches /
 // one: 768 x 2048 and 2048 x 2048 Q4_0 5.95 / 5.50 and 6.03 / 5.57, Q4_K 5.51
 // / 5.14 and 5.50 / 5.18; 8192 x 2048 (1024 work groups) Q4_K 6.36 / 7.12;
-// 4096 x 4096 6.61 / 7.72; two vectors per group 768 x 2048 6.03 / 6.51.
+// 4096 x 4096 6.61 / 7.72; two vectors per group 768 x 2048 6.03 / 6.51.  With the
+// FFN norm, us per layer of a dense one-lane frame, Q4_0 (Q8_0): ffn 3584 (448
+// work groups) over 4096 columns 60.1 / 59.3 (68.3 / 68.4), 4608 (576) 63.8 / 64.5
+// (77.5 / 78.5), 5120 (640) 64.7 / 65.9, 8192 (1024) 70.7 / 82.1; 5120 over 2048
+// columns 53.6 / 52.4 (62.8 / 62.2), 8192 57.4 / 56.3.
 constexpr int SELF_MAX_COLS = 2048, SELF_MAX_WGS = 512, SELF_MAX_WGS_NORM = 640;
 bool launch_dmmv_self(bool fused, DmmvSegParams sp, const float *x, int x_stride, const float *norm_w, float eps,
                       hipStream_t st) {
@@ -307,7 +311,7 @@ bool launch_dmmv_self(bool fused, DmmvSegParams sp, const float *x, int x_stride
     }
     part = align16(part);
     const size_t lds = part + self_act_bytes(cols);
-    const long wgs = (long)tiles * sp.base.n_groups, max_wgs = norm_w ? SELF_MAX_WGS_NORM : SELF_MAX_WGS;
+    const long wgs = (long)tiles * sp.base.n_groups, max_wgs = norm_w && cols <= SELF_MAX_COLS ? SELF_MAX_WGS_NORM : SELF_MAX_WGS;
     if (lds > 64 * 1024 || ((!norm_w || fused) && wgs > max_wgs)) // (the q/k/v launch: at any size)
         return false;
     const dim3 grid(tiles, sp.base.n_groups);

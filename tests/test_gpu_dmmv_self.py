@@ -112,3 +112,31 @@ def test_one_timing_record_per_frame_stage(n):
         assert [st[k]["count"] for k in ("qkv", "wo", "dense")] == [layers] * 3
     finally:
         be.profileKernels(False)
+
+
+@pytest.mark.parametrize("dim,ffn,launches", [(2048, 5120, 0), (2048, 5152, 1), (2304, 4096, 0), (2304, 4128, 1)])
+def test_ffn_norm_with_gate_up_at_its_limits(oracle, dim, ffn, launches):
+    """One lane, PARITY: the FFN norm inside the gate/up launch up to 640 work
+    groups over 2048 columns and 512 over more, in a launch of its own beyond
+    (one more per layer).  Logits bit-identical to the oracle's step."""
+    import dataclasses
+
+    import loom_amd
+    from loom_amd import frame as lh
+    from oracle.model import OracleModel
+    from test_gpu_frame import _batch_steps
+
+    loom_amd.init(0)
+    layers = 2
+    spec = dataclasses.replace(lh.stories15m(ctx_len=32), dim=dim, n_layers=layers, vocab=512, n_heads=4,
+                               n_kv_heads=4, head_dim=64, rope_dim=64, ffn=ffn)
+    dm = lh.DeviceModel.synth(spec, seed=5, keep_ggml=True)
+    rels, same = _batch_steps(lh, OracleModel(oracle, dm), dm, 1, 2, 8, seed=3)
+    assert rels.max() == 0.0 and same
+    count = []
+    for f in (4096, ffn):
+        dec = lh.Decoder(lh.DeviceModel.synth(dataclasses.replace(spec, ffn=f), seed=5), 1)
+        loom_amd.take_launch_count()
+        assert dec.step() == loom_amd.OK
+        count.append(loom_amd.take_launch_count())
+    assert count[1] - count[0] == launches * layers
