@@ -201,9 +201,9 @@ __global__ __launch_bounds__(256) void dmmv_seg_kernel(DmmvSegParams sp) {
     }
 }
 
-// ---- one vector per group: its int8 form made by the matvec's own work groups -----
+// ---- one vector: its int8 form made by the matvec's own work groups ---------------
 // A matvec of one vector is a chain of short launches, quant_act's 2.3 us and
-// dmmv's 4.5 at 768 x 2048.  Here every work group quantizes its group's
+// dmmv's 4.5 at 768 x 2048.  Here every work group quantizes the
 // vector into LDS and runs the tile against it: one launch, and no round trip
 // of the int8 row.  NORM: x is first normalised by the reference's rmsnorm
 // (the sequential sum of the squares, 4 waves), every work group for itself --
@@ -212,7 +212,9 @@ __global__ __launch_bounds__(256) void dmmv_seg_kernel(DmmvSegParams sp) {
 // matvec call from Python 10.8 -> 7.4 us at 768 x 2048 (the kernel alone 6.1 to
 // 6.7 us up to 2048 x 2048, where the two took 4.6 and 4.7 to 5.1).  Same values
 // as norm_quant_kernel / quant_act_kernel followed by dmmv_seg_kernel or
-// dmmv_kernel.
+// dmmv_kernel.  One group is launched; the kernel still indexes by it, as the
+// same kernel with the group and the vector's stride fixed took the stories15M
+// token from 231 to 235 us.
 constexpr int NSEG_MAX_DIM = 4096;
 constexpr int NSEG_XV = norm_xv(NSEG_MAX_DIM, 4);
 
@@ -278,14 +280,14 @@ __global__ __launch_bounds__(256, 4) void dmmv_self_kernel(DmmvSegParams sp, con
     }
 }
 
-// Up to DMMV_MAX_SEG matrices (or one fused pair, base.w2) against groups of
-// one of the vectors x; norm_w: one group, normalised first.  False = not
-// served (nothing launched; the caller quantizes apart): LDS, rows so long or
+// Up to DMMV_MAX_SEG matrices (with norm_w also one fused pair, base.w2) against
+// one vector (base.groups: one group of one); norm_w: normalised first.  False =
+// not served (nothing launched; the caller quantizes apart): LDS, rows so long or
 // work groups so many that each one's repeated quantization (or norm) costs
 // more than the launch it saves.  Measured, us back to back, two launches /
 // one: 768 x 2048 and 2048 x 2048 Q4_0 5.95 / 5.50 and 6.03 / 5.57, Q4_K 5.51
 // / 5.14 and 5.50 / 5.18; 8192 x 2048 (1024 work groups) Q4_K 6.36 / 7.12;
-// 4096 x 4096 6.61 / 7.72; two vectors per group 768 x 2048 6.03 / 6.51.  With the
+// 4096 x 4096 6.61 / 7.72; two vectors at 768 x 2048 6.03 / 6.51.  With the
 // FFN norm, us per layer of a dense one-lane frame, Q4_0 (Q8_0): ffn 3584 (448
 // work groups) over 4096 columns 60.1 / 59.3 (68.3 / 68.4), 4608 (576) 63.8 / 64.5
 // (77.5 / 78.5), 5120 (640) 64.7 / 65.9, 8192 (1024) 70.7 / 82.1; 5120 over 2048
@@ -294,8 +296,8 @@ constexpr int SELF_MAX_COLS = 2048, SELF_MAX_WGS = 512, SELF_MAX_WGS_NORM = 640;
 bool launch_dmmv_self(bool fused, DmmvSegParams sp, const float *x, int x_stride, const float *norm_w, float eps,
                       hipStream_t st) {
     const int cols = sp.base.cols;
-    if (sp.n_seg < 1 || (fused && sp.n_seg != 1) || sp.base.n_groups_dev ||
-        (norm_w ? sp.base.n_groups != 1 || cols > NSEG_MAX_DIM || cols % 32 : cols > SELF_MAX_COLS))
+    if (sp.n_seg < 1 || (fused && (sp.n_seg != 1 || !norm_w)) || sp.base.n_groups_dev || sp.base.n_groups != 1 ||
+        (norm_w ? cols > NSEG_MAX_DIM || cols % 32 : cols > SELF_MAX_COLS))
         return false;
     size_t part = 0;
     int tiles = 0;
@@ -311,13 +313,11 @@ bool launch_dmmv_self(bool fused, DmmvSegParams sp, const float *x, int x_stride
     }
     part = align16(part);
     const size_t lds = part + self_act_bytes(cols);
-    const long wgs = (long)tiles * sp.base.n_groups, max_wgs = norm_w && cols <= SELF_MAX_COLS ? SELF_MAX_WGS_NORM : SELF_MAX_WGS;
-    if (lds > 64 * 1024 || ((!norm_w || fused) && wgs > max_wgs)) // (the q/k/v launch: at any size)
+    const int max_wgs = norm_w && cols <= SELF_MAX_COLS ? SELF_MAX_WGS_NORM : SELF_MAX_WGS;
+    if (lds > 64 * 1024 || ((!norm_w || fused) && tiles > max_wgs)) // (the q/k/v launch: at any size)
         return false;
-    const dim3 grid(tiles, sp.base.n_groups);
-    auto kern = norm_w ? (fused ? dmmv_self_kernel<true, true> : dmmv_self_kernel<false, true>)
-                       : (fused ? dmmv_self_kernel<true, false> : dmmv_self_kernel<false, false>);
-    hipLaunchKernelGGL(kern, grid, dim3(256), lds, st, sp, x, x_stride, norm_w, eps, (int)part);
+    auto kern = fused ? dmmv_self_kernel<true, true> : norm_w ? dmmv_self_kernel<false, true> : dmmv_self_kernel<false, false>;
+    hipLaunchKernelGGL(kern, dim3(tiles), dim3(256), lds, st, sp, x, x_stride, norm_w, eps, (int)part);
     note_launch();
     return true;
 }

@@ -62,9 +62,9 @@ struct DmmvSegParams {
     int n_seg;
 };
 bool launch_dmmv_seg(int nt, DmmvSegParams sp, hipStream_t st);
-// The same, and a fused pair (base.w2), for groups of one f32 vector each that
-// the launch quantizes itself; norm_w: one group, the PARITY rmsnorm of x
-// applied first.  False = not served (nothing launched).
+// The same for one f32 vector (one group) that the launch quantizes itself, so no
+// output may overlap it; norm_w: the PARITY rmsnorm of x applied first, then also
+// a fused pair (base.w2).  False = not served (nothing launched).
 bool launch_dmmv_self(bool fused, DmmvSegParams sp, const float *x, int x_stride, const float *norm_w, float eps,
                       hipStream_t st);
 
