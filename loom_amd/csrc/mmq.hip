@@ -969,9 +969,9 @@ static bool mmq_shape(int rows, int cols, int mt, bool fused, int &rg, int &ks, 
 }
 
 // ---- Q8_0 / Q4_0 (32-value blocks) on the int8 matrix cores ----------------------
-// A work group of MQ32_W waves per (16-row tile, 16 tokens of a group: a group
-// of up to 32 takes two, along z); wave w takes the w-th share of the rows'
-// 64-value spans.  Per span
+// Lane groups (consecutive vectors) of matrices that leave the streamed kernel
+// too few waves.  A work group of MQ32_W waves per (16-row tile, 16 vectors);
+// wave w takes the w-th share of the rows' 64-value spans.  Per span
 // (blocks 2s and 2s + 1) lane quarter q4 holds 16 values of block 2s + q4/2
 // -- A: token r16's activations, B: row r16's quants (Q4_0 as nibble - 8) --
 // and two MFMAs over the span, each with the other block's quarters of the
@@ -989,61 +989,33 @@ constexpr int MQ32_PART = 32768;  // LDS floats of block values: nb * 256
 
 template <int T>
 __global__ __launch_bounds__(64 * MQ32_W) void mmq32_kernel(DmmvParams p) {
-    constexpr int MT = 1;
     static_assert(T == LH_Q8_0 || T == LH_Q4_0, "32-value blocks");
     constexpr int QB = T == LH_Q8_0 ? 32 : 16; // quant bytes per block
-    constexpr int NO = 256 * MT;               // outputs per work group: (token, row)
+    constexpr int NO = 256;                    // outputs per work group: (token, row)
     constexpr int MAXNB = 64 * MQ32_W * MQ32_MAXS / 32;
     __shared__ __align__(16) float part[MQ32_PART];      // [block][token * 16 + row]
-    __shared__ __align__(16) float xds[16 * MT][MAXNB];  // the tokens' block scales
+    __shared__ __align__(16) float xds[16][MAXNB];       // the tokens' block scales
     const int ln = threadIdx.x & 63, r16 = ln & 15, q4 = ln >> 4;
     const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
-    const bool ident = p.ident_n > 0;
-    DmmvGroup grp;
-    if (ident) {
-        grp.plane = 0;
-        grp.first = (int)blockIdx.y * 16;
-        grp.n = min(16, p.ident_n - grp.first);
-    } else {
-        const int ng = p.n_groups_dev ? *p.n_groups_dev : p.n_groups;
-        if ((int)blockIdx.y >= ng)
-            return;
-        grp = p.groups[blockIdx.y];
-        // tokens 16 z .. of the group (pairs first + 16 z ..)
-        grp.first += 16 * (int)blockIdx.z;
-        grp.n = min(16, grp.n - 16 * (int)blockIdx.z);
-        if (grp.n <= 0)
-            return;
-    }
-    const int n = grp.n, cols = p.cols, nb = cols / 32, ns = cols / 64;
+    const int first = (int)blockIdx.y * 16; // this group's vectors: first .. first + n - 1
+    const int n = min(16, p.ident_n - first), cols = p.cols, nb = cols / 32, ns = cols / 64;
     const int s_lo = wave * ns / MQ32_W, cnt = (wave + 1) * ns / MQ32_W - s_lo; // this wave's spans
     const int row0 = (int)blockIdx.x * 16;
     const int row = min(row0 + r16, p.rows - 1);
     const size_t U = (size_t)p.rows * nb;
-    const uint8_t *wb = p.w + (size_t)grp.plane * p.plane_bytes;
-    // A row r16 of token tile mt carries a vector (tokens past n repeat the
-    // last; their outputs are never stored); this lane's outputs are tokens
-    // 16 mt + 4 q4 + i of row r16
-    const int8_t *xr[MT];
-#pragma unroll
-    for (int mt = 0; mt < MT; mt++) {
-        const int tk = min(16 * mt + r16, n - 1);
-        const int vrow = ident ? grp.first + tk : p.pair_src[grp.first + tk];
-        xr[mt] = p.xq + (size_t)vrow * cols + 16 * q4;
-    }
+    const uint8_t *wb = p.w;
+    // A row r16 carries a vector (tokens past n repeat the last; their outputs are
+    // never stored); this lane's outputs are tokens 4 q4 + i of row r16
+    const int8_t *xr = p.xq + (size_t)(first + min(r16, n - 1)) * cols + 16 * q4;
     // the group's block scales, bound for LDS (row tk of xds: token tk's nb
     // scales; tokens past n repeat the last): thread (tk, part) loads blocks
     // xpart + TPT u of token tk, unconditionally from clamped indices, first;
     // they are stored after the first spans' loads are out, so that store
     // waits for these loads alone
-    constexpr int TPT = 64 * MQ32_W / (16 * MT); // threads per token
-    constexpr int XU = (MAXNB + TPT - 1) / TPT;  // scales per thread (at most)
+    constexpr int TPT = 64 * MQ32_W / 16;       // threads per token
+    constexpr int XU = (MAXNB + TPT - 1) / TPT; // scales per thread (at most)
     const int xtk = (int)threadIdx.x / TPT, xpart = (int)threadIdx.x % TPT;
-    const float *xdr;
-    {
-        const int tc = min(xtk, n - 1);
-        xdr = p.xd + (size_t)(ident ? grp.first + tc : p.pair_src[grp.first + tc]) * nb;
-    }
+    const float *xdr = p.xd + (size_t)(first + min(xtk, n - 1)) * nb;
     float xe[XU];
 #pragma unroll
     for (int u = 0; u < XU; u++)
@@ -1054,7 +1026,7 @@ __global__ __launch_bounds__(64 * MQ32_W) void mmq32_kernel(DmmvParams p) {
     const uint8_t *wq = wb + ((size_t)row * nb + (q4 >> 1)) * QB + (T == LH_Q8_0 ? 16 * (q4 & 1) : 0);
     const uint32_t *wd = (const uint32_t *)(wb + U * QB + (size_t)row * nb * 2);
     struct Span {
-        mmq_i4 a[MT], w;
+        mmq_i4 a, w;
         uint32_t d;
     };
     // span j of this wave (past its last: the last, loaded and not used)
@@ -1062,9 +1034,7 @@ __global__ __launch_bounds__(64 * MQ32_W) void mmq32_kernel(DmmvParams p) {
         const int sc = s_lo + min(j, cnt - 1);
         o.w = *(const mmq_i4 *)(wq + (size_t)2 * sc * QB);
         o.d = wd[sc];
-#pragma unroll
-        for (int mt = 0; mt < MT; mt++)
-            o.a[mt] = *(const mmq_i4 *)(xr[mt] + 64 * sc);
+        o.a = *(const mmq_i4 *)(xr + 64 * sc);
     };
     const mmq_i4 z = {0, 0, 0, 0};
     const bool lo = q4 < 2;
@@ -1079,19 +1049,16 @@ __global__ __launch_bounds__(64 * MQ32_W) void mmq32_kernel(DmmvParams p) {
         }
         const mmq_i4 wa = lo ? wv : z, wbk = lo ? z : wv;
         const float dwa = half_bits_to_float(o.d & 0xffffu), dwb = half_bits_to_float(o.d >> 16);
+        const mmq_i4 da = __builtin_amdgcn_mfma_i32_16x16x64_i8(o.a, wa, z, 0, 0, 0);
+        const mmq_i4 db = __builtin_amdgcn_mfma_i32_16x16x64_i8(o.a, wbk, z, 0, 0, 0);
 #pragma unroll
-        for (int mt = 0; mt < MT; mt++) {
-            const mmq_i4 da = __builtin_amdgcn_mfma_i32_16x16x64_i8(o.a[mt], wa, z, 0, 0, 0);
-            const mmq_i4 db = __builtin_amdgcn_mfma_i32_16x16x64_i8(o.a[mt], wbk, z, 0, 0, 0);
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const int tk = 16 * mt + 4 * q4 + i;
-                const float2 xd = *(const float2 *)&xds[tk][2 * sc];
-                const float sa = dwa * xd.x;
-                part[(size_t)(2 * sc) * NO + tk * 16 + r16] = sa * (float)da[i];
-                const float sb = dwb * xd.y;
-                part[(size_t)(2 * sc + 1) * NO + tk * 16 + r16] = sb * (float)db[i];
-            }
+        for (int i = 0; i < 4; i++) {
+            const int tk = 4 * q4 + i;
+            const float2 xd = *(const float2 *)&xds[tk][2 * sc];
+            const float sa = dwa * xd.x;
+            part[(size_t)(2 * sc) * NO + tk * 16 + r16] = sa * (float)da[i];
+            const float sb = dwb * xd.y;
+            part[(size_t)(2 * sc + 1) * NO + tk * 16 + r16] = sb * (float)db[i];
         }
     };
     // each span's loads are issued as a unit, in span order (the fences keep
@@ -1125,31 +1092,25 @@ __global__ __launch_bounds__(64 * MQ32_W) void mmq32_kernel(DmmvParams p) {
         for (int bl = 0; bl < nb; bl++)
             acc = acc + part[(size_t)bl * NO + o];
         if (tk < n && row0 + rr < p.rows) {
-            const int dst = ident ? grp.first + tk : p.pair_dst[grp.first + tk];
-            float *out = p.out + (size_t)dst * p.out_stride + row0 + rr;
+            float *out = p.out + (size_t)(first + tk) * p.out_stride + row0 + rr;
             *out = p.accumulate ? *out + acc : acc;
         }
     }
 }
 
-static bool mmq32_supported(int t, int cols, int max_tok, bool fused) {
+static bool mmq32_supported(int t, int cols, bool fused) {
     // the block values of a work group fill (cols / 32) * 256 floats of LDS
     return (t == LH_Q8_0 || t == LH_Q4_0) && !fused && cols % 64 == 0 && cols >= 64 * MQ32_W &&
-           cols <= 64 * MQ32_W * MQ32_MAXS && max_tok >= 1 && max_tok <= 32 &&
-           (size_t)(cols / 32) * 256 <= (size_t)MQ32_PART;
+           cols <= 64 * MQ32_W * MQ32_MAXS && (size_t)(cols / 32) * 256 <= (size_t)MQ32_PART;
 }
 
-// Identity pairs go in groups of 16 tokens; a caller's groups of up to 32
-// take two work groups each (z).
-static bool launch_mmq32(int t, int max_tok, const DmmvParams &p, hipStream_t st) {
-    const bool ident = p.ident_n > 0;
-    const int groups = ident ? (p.ident_n + 15) / 16 : p.n_groups;
-    const dim3 grid((p.rows + 15) / 16, groups, ident || max_tok <= 16 ? 1 : 2), block(64 * MQ32_W);
+// p.ident_n vectors in groups of 16.
+static void launch_mmq32(int t, const DmmvParams &p, hipStream_t st) {
+    const dim3 grid((p.rows + 15) / 16, (p.ident_n + 15) / 16), block(64 * MQ32_W);
     if (t == LH_Q8_0)
         hipLaunchKernelGGL(mmq32_kernel<LH_Q8_0>, grid, block, 0, st, p);
     else
         hipLaunchKernelGGL(mmq32_kernel<LH_Q4_0>, grid, block, 0, st, p);
-    return true;
 }
 
 // ---- many vectors: a 64-row x 128-vector tile per work group -----------------------
@@ -1711,7 +1672,7 @@ static bool is_k(int t) { return t == LH_Q4_K || t == LH_Q6_K; }
 // 32-value blocks in mmq32_kernel's.
 static bool mmq_oneshot(int t, int cols, int max_tok, bool fused) {
     if (!is_k(t))
-        return mmq32_supported(t, cols, max_tok, fused);
+        return mmq32_supported(t, cols, fused);
     if (cols % 256 || cols < 256 || max_tok < 1 || max_tok > 32)
         return false;
     if (fused && t != LH_Q4_K) // a fused pair is gate/up: Q4_K only here
@@ -1817,7 +1778,7 @@ static bool lanes_tiled(int t, int rows, int cols, int n) {
 //     56.5, Q4_0 47.9 / 58.2; at 32, 512 pairs, 111 / 57 and 84 / 59).
 static bool lanes32_on_cores(int t, int rows, int cols, int n) {
     const size_t size = (size_t)rows * cols;
-    if (mmq32_supported(t, cols, 16, false)) {
+    if (mmq32_supported(t, cols, false)) {
         if (n < 8)
             return n >= 5 && size >= ((size_t)8 << 20);
         const bool line = cols / 32 * (t == LH_Q8_0 ? 32 : 16) % 128 == 0;
@@ -1979,8 +1940,10 @@ bool launch_mmq(int t, int max_tok, bool fused, const DmmvParams &p, hipStream_t
         return false;
     const int mt = max_tok > 16 ? 2 : 1;
     if (!is_k(t)) {
+        if (!stream && p.ident_n <= 0) // mmq32_kernel takes lane groups only
+            return false;
         if (!stream)
-            launch_mmq32(t, max_tok, p, st);
+            launch_mmq32(t, p, st);
         else if (t == LH_Q8_0)
             fused ? mmw32_launch_t<LH_Q8_0, true>(p, st) : mmw32_launch_t<LH_Q8_0, false>(p, st);
         else
