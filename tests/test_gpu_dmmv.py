@@ -132,11 +132,12 @@ def test_matmul_bit_exact_to_per_vector_oracle(be, oracle, t):
 @pytest.mark.parametrize("t", [Q4_K, Q6_K, Q8_0, Q4_0])
 @pytest.mark.parametrize("rows,cols", [(37, 768), (300, 4096), (64, 256), (130, 2048)])
 def test_matmul_matrix_cores_bit_exact(be, oracle, t, rows, cols):
-    """From 16 vectors on, Q4_K / Q6_K matmuls run on the int8 matrix cores
-    (mmq.hip, groups of 32), and so do Q8_0 / Q4_0 over whole 64-value spans
-    (mmq32_kernel: a wave per 16-row tile walks the blocks in order, 16 vectors
-    a group): bit-identical to per-vector oracle matvecs, including ragged row
-    tiles and groups."""
+    """From 16 vectors on, these Q4_K / Q6_K matmuls run on the int8 matrix cores
+    (mmq_kernel, groups of 16 and 32), and so do Q8_0 / Q4_0 300 x 4096 and Q8_0
+    130 x 2048 (mmq32_kernel: eight waves share a 16-row tile's spans, 16 vectors
+    a group); the smaller Q8_0 / Q4_0 ones stay on the dot4 matvec.
+    Bit-identical to per-vector oracle matvecs, including ragged row tiles and
+    groups."""
     rng = np.random.default_rng(77 + t + rows)
     raw = npref.pinned_scale_blocks(t, rows, cols, rng)
     for n in (16, 17, 32, 45):

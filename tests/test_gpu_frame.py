@@ -244,16 +244,19 @@ def test_llama_frame_batch_head_layouts(lh, oracle, heads):
 
 @pytest.mark.parametrize("wt", [2, 8])  # Q4_0, Q8_0
 @pytest.mark.parametrize("n", [16, 32])
-def test_llama_frame_batch_32_block_matrix_cores(lh, oracle, wt, n):
+@pytest.mark.parametrize("heads,ffn,vocab", [((8, 4), 1024, 2048), ((18, 6), 4096, 4096)])
+def test_llama_frame_batch_32_block_matrix_cores(lh, oracle, wt, n, heads, ffn, vocab):
     """A llama-architecture model 512 wide in Q4_0 or Q8_0 throughout (q, k,
-    v, wo, the FFN and the head): from 16 lanes every one of its matmuls runs
-    on mmq32_kernel (whole 64-value spans, 512 to 4096 columns) through the
-    frame.  PARITY per-lane logits against lo_decode_batch over 3 steps on
-    identical state, identical greedy tokens."""
+    v, wo, the FFN and the head).  The small one stays on the dot4 matvec.  The
+    wider one's wo (512 x 1152) and FFN down (512 x 4096) run on mmq32_kernel
+    with their residual adds, its head (4096 x 512, from 20 lanes) on
+    mmw32_kernel, and at 32 lanes so does the fused gate/up.  PARITY per-lane
+    logits against lo_decode_batch over 3 steps on identical state, identical
+    greedy tokens."""
     import dataclasses
 
-    spec = dataclasses.replace(lh.stories15m(ctx_len=160), dim=512, n_layers=2, vocab=2048, n_heads=8,
-                               n_kv_heads=4, head_dim=64, rope_dim=64, ffn=1024, embed_t=wt, output_t=wt,
+    spec = dataclasses.replace(lh.stories15m(ctx_len=160), dim=512, n_layers=2, vocab=vocab, n_heads=heads[0],
+                               n_kv_heads=heads[1], head_dim=64, rope_dim=64, ffn=ffn, embed_t=wt, output_t=wt,
                                wq_t=wt, wk_t=wt, wv_t=wt, wo_t=wt, ffn_gate_t=wt, ffn_down_t=wt)
     dm = lh.DeviceModel.synth(spec, seed=31 + wt, keep_ggml=True)
     om = OracleModel(oracle, dm)

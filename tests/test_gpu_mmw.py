@@ -1,6 +1,6 @@
-"""GPU parity of the matrix-core matmul that streams a row's blocks in order
-(mmw_kernel, mmq.hip) and of the one with 64 x 128 tiles (mmp_kernel):
-bit-exact against per-vector oracle matvecs at the edges of its row tiles (16
+"""GPU parity of the matrix-core matmuls that stream a row's blocks in order
+(mmw_kernel and, for 32-value blocks, mmw32_kernel, mmq.hip), of the one with 64
+x 128 tiles (mmp_kernel) and of the one-shot kernels beside them: bit-exact against per-vector oracle matvecs at the edges of its row tiles (16
 rows, 64 per work group), token sets (8) and groups (16, 32), block counts (odd
 and even, with the tokens' rows staged in LDS up to 2048 columns and not
 beyond), and at the extreme integers of its f16 mins and two-digit scales.
@@ -107,11 +107,12 @@ Q4_0, Q8_0 = 2, 8
 
 
 # lane groups of 32-value blocks that stream: at least 768 (row tile, 16 vectors)
-# pairs, or a shape the one-shot kernel does not hold
+# pairs, or a shape the one-shot kernel does not hold with enough rows x vectors
+# (1100 x 1952 from 58 vectors, the dot4 matvec below)
 @pytest.mark.parametrize("t", [Q4_0, Q8_0])
 @pytest.mark.parametrize("rows,cols,n", [(8192 + 5, 288, 16), (8192 + 17, 2080, 20), (12288 + 1, 2048, 9),
                                          (12288 + 15, 4096, 16), (16384, 32, 65), (8192 + 33, 4384, 33),
-                                         (1100, 1952, 8)])
+                                         (1100, 1952, 8), (1100, 1952, 58)])
 def test_streamed_32_block_matmul_edges(be, oracle, t, rows, cols, n):
     """Odd block counts (9, 65, 137, 61), units of fewer than 8 blocks, one
     block per row, partial token sets and groups, rows staged whole and not."""
@@ -146,9 +147,10 @@ def test_k_quant_routes(be, oracle, t, rows, cols, n):
     _check(be, oracle, t, raw, xs, rows, cols)
 
 
-# five to fifteen vectors on the matrix cores (one-shot), rows too wide for 32 lanes a wave
+# five to fifteen vectors on the matrix cores (one-shot; 1100 x 1024 Q4_0 on the dot4 matvec), rows too wide for
+# 32 lanes a wave
 @pytest.mark.parametrize("t,rows,cols,n", [(Q4_K, 300, 2048, 5), (Q4_K, 77, 8192, 17), (Q6_K, 300, 768, 8),
-                                           (Q6_K, 130, 8192, 9), (Q8_0, 2100, 4096, 5), (Q4_0, 1100, 1024, 11),
+                                           (Q6_K, 130, 8192, 9), (Q8_0, 2100, 4096, 5), (Q4_0, 1100, 1024, 11), (Q4_0, 1100, 1088, 11),
                                            (Q4_K, 4100, 11008, 32), (Q6_K, 8200, 8448, 16)])
 def test_matmul_from_five_vectors(be, oracle, t, rows, cols, n):
     rng = np.random.default_rng(rows + cols + n + t)
@@ -214,3 +216,40 @@ def test_widest_streamed_rows(be, oracle, t, cols, served):
     for k in (0, 100, n - 1):
         want = oracle.matvec(t, raw, x[k].cpu().numpy(), rows, cols)
         assert np.array_equal(out[k].cpu().numpy().view(np.uint32), want.view(np.uint32)), k
+
+
+# the shared expert's matmuls add to the routed sum (accumulate) and run as one matrix each
+@pytest.mark.parametrize("gt,dt,dim,sffn,n", [
+    (Q8_0, Q8_0, 2048, 288, 17), (Q4_0, Q4_0, 2048, 288, 17),   # down streamed, 32-value blocks
+    (Q8_0, Q8_0, 288, 4096, 32), (Q4_0, Q4_0, 288, 4096, 32),   # gate/up streamed as a pair, rows staged; down one-shot
+    (Q8_0, Q8_0, 2080, 4096, 33), (Q4_0, Q4_0, 2080, 4096, 33),  # the same, rows not staged
+    (Q4_K, Q4_K, 8192, 256, 16), (Q4_K, Q6_K, 8192, 256, 16),   # down one-shot
+    (Q4_K, Q4_K, 8192, 256, 24), (Q4_K, Q6_K, 8192, 256, 24),   # down streamed, in groups of 16 and 32
+    (Q4_K, Q4_K, 8192, 256, 250), (Q4_K, Q6_K, 8192, 256, 250),  # down on 64 x 128 tiles
+])
+def test_shared_expert_adds_on_matrix_cores(be, oracle, gt, dt, dim, sffn, n):
+    """Bits of the whole layer against lo_moe_batch_union (EXPERT_ASC adds the
+    routed sum to what out holds, then the shared expert's)."""
+    import torch
+    from test_gpu_moe import make_layer
+
+    ffn, E, k = 256 if gt == Q4_K else 96, 4, 1
+    w = make_layer(oracle, dim, ffn, E, k, seed=dim + n, gate_t=gt, down_t=dt)
+    rng = np.random.default_rng(dim + sffn + n)
+    sg, su = (npref.pinned_scale_blocks(gt, sffn, dim, rng) for _ in range(2))
+    sd = npref.pinned_scale_blocks(dt, dim, sffn, rng)
+    w.shexp = (sg, su, sd, gt, gt, dt, sffn)
+
+    def dev(t, raw, rows, cols, planes=1):
+        return be.repack_dev(t, torch.from_numpy(raw).cuda(), rows, cols, planes)
+
+    layer = be.MoeLayer(dim, ffn, E, k, torch.from_numpy(w.router).cuda(), dev(gt, w.gate, ffn, dim, E),
+                        dev(gt, w.up, ffn, dim, E), dev(dt, w.down, dim, ffn, E), gt, gt, dt,
+                        shexp=(dev(gt, sg, sffn, dim), dev(gt, su, sffn, dim), dev(dt, sd, dim, sffn), gt, gt, dt, sffn))
+    xs = np.stack([oracle.normal(dim, 700 + i, 0.0, 1.0) for i in range(n)])
+    resid = np.stack([oracle.normal(dim, 900 + i, 0.0, 1.0) for i in range(n)])
+    out = torch.from_numpy(resid.copy()).cuda()
+    layer(torch.from_numpy(xs).cuda(), out, combine=be.COMBINE_EXPERT_ASC)
+    want, _, _ = oracle.moe_batch_union(w, xs, resid)
+    torch.cuda.synchronize()
+    assert np.array_equal(out.cpu().numpy().view(np.uint32), want.view(np.uint32))

@@ -261,13 +261,13 @@ def test_moe_layer_dev_gatings_and_down_types(be, oracle, down_t, ffn, gi, n):
 @pytest.mark.parametrize("down_t,ffn", [(Q8_0, 512), (Q4_0, 768), (Q8_0, 4096)])
 @pytest.mark.parametrize("n", [16, 32])
 def test_moe_layer_dev_matrix_core_32_block_downs(be, oracle, down_t, ffn, n):
-    """From 16 tokens the batched path runs the expert matmuls on the int8
-    matrix cores: the fused Q4_K gate/up on mmq.hip's K-quant kernels and a
-    Q8_0 / Q4_0 down on mmq32_kernel in its grouped form (expert planes, the
-    groups' pair sources and destinations; ffn 4096 is its widest span
-    count).  8 experts top-4, so at 32 tokens the busiest experts take more
-    than one group of 16.  Ids, gates and the layer's output bits against
-    lo_moe_batch_union."""
+    """The batched path with its expert matmuls on the int8 matrix cores: the
+    fused Q4_K gate/up on mmq.hip's K-quant kernels and a Q8_0 / Q4_0 down on
+    mmw32_kernel in its grouped form (expert planes, the groups' pair
+    destinations; ffn 4096 past its staged rows) -- at 32 tokens, and for ffn 4096
+    at 16; the smaller two at 16 tokens on the grouped dot4 matvec.  8 experts
+    top-4, so at 32 tokens the busiest experts take more than one group of 16.
+    Ids, gates and the layer's output bits against lo_moe_batch_union."""
     import torch
 
     dim, E, k = 512, 8, 4

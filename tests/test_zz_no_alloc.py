@@ -12,7 +12,7 @@ from test_gpu_moe import _dev_layer, make_layer
 
 pytestmark = pytest.mark.gpu
 
-Q4_K, Q6_K = 12, 14
+Q8_0, Q4_K, Q6_K = 8, 12, 14
 
 
 @pytest.fixture(scope="module")
@@ -59,6 +59,34 @@ def test_noalloc_matches_allocating_entry_point(be, oracle):
         torch.cuda.synchronize()
         assert torch.equal(ids_a, ids_b), n
         assert np.array_equal(out_a.cpu().numpy().view(np.uint32), out_b.cpu().numpy().view(np.uint32)), n
+
+
+@pytest.mark.parametrize("gate_t,down_t", [(Q4_K, Q6_K), (Q8_0, Q8_0)])
+def test_noalloc_without_room_for_the_groups_token_rows(be, oracle, gate_t, down_t):
+    """248 tokens of 1024 x 768 x 64 top-8 need 6176 B less than the array holds,
+    and the table of the groups' token rows takes 12032 B: it is left out, and
+    the streamed matmuls find their rows through the pairs.  Bit-identical to
+    the allocating entry point, which has the table; one token more is refused."""
+    import torch
+
+    import loom_amd
+    from loom_amd import COMBINE_EXPERT_ASC
+
+    n, dim, k = 248, 1024, 8
+    w = make_layer(oracle, dim, 768, 64, k, seed=73, gate_t=gate_t, down_t=down_t)
+    layer = _dev_layer(be, w)
+    g = torch.Generator(device="cuda").manual_seed(6)
+    x = torch.randn(n + 1, dim, generator=g, device="cuda")
+    out_a = torch.zeros(n, dim, device="cuda")
+    out_b = torch.zeros(n, dim, device="cuda")
+    assert _call("loomhip_moe_layer_dev", layer, x[:n], out_a, COMBINE_EXPERT_ASC, None) == loom_amd.OK
+    rc = _call("loomhip_moe_layer_dev_noalloc", layer, x[:n], out_b, COMBINE_EXPERT_ASC, None)
+    assert rc == loom_amd.OK, loom_amd.last_error()
+    torch.cuda.synchronize()
+    assert bool((out_a != 0).any())
+    assert np.array_equal(out_a.cpu().numpy().view(np.uint32), out_b.cpu().numpy().view(np.uint32))
+    out_c = torch.zeros(n + 1, dim, device="cuda")
+    assert _call("loomhip_moe_layer_dev_noalloc", layer, x, out_c, COMBINE_EXPERT_ASC, None) == loom_amd.ERR_ARG
 
 
 def test_noalloc_refuses_a_workspace_beyond_the_array(be, oracle):
