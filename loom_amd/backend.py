@@ -193,19 +193,21 @@ def profileKernels(enable: bool) -> None:
 
 
 _KERNEL_SYMBOLS = {
-    "gate_up": "moe_gateup_decode_kernel (n <= 4) / dmmv_kernel<T, NT, FUSED=true> / from 5 to 20 tokens, by type "
-               "and size, mmw_kernel<T, 1, true, ...> or mmw32_kernel<T, true, ...> (grouped gate/up + SwiGLU)",
+    "gate_up": "moe_gateup_decode_kernel (n <= 4) / dmmv_kernel<T, NT, FUSED=true> / from 5 tokens or more, by type "
+               "and size, mmq_kernel<T, 1, true, SBW>, mmw_kernel<T, 1, true, ...> or mmw32_kernel<T, true, ...> "
+               "(grouped gate/up + SwiGLU)",
     "down": "moe_down_decode_kernel (n <= 4) / dmmv_kernel<T, NT, FUSED=false> / as gate_up "
-            "mmw_kernel<T, 1, false, ...> or mmw32_kernel<T, false, ...> (grouped down)",
-    "dense": "dmmv_self_kernel or dmmv_kernel<T, NT, false> / from 5 to 8 vectors, by type, mmq_kernel, mmq32_kernel, "
-             "mmw_kernel, mmw32_kernel or mmp_kernel by size (dense matvec and matmul)",
+            "mmq_kernel<T, 1, false, SBW>, mmw_kernel<T, 1, false, ...> or mmw32_kernel<T, false, ...> (grouped down)",
+    "dense": "dmmv_self_kernel or dmmv_kernel<T, NT, false> / from 5 vectors or more, by type and size, mmq_kernel, "
+             "mmq32_kernel, mmw_kernel, mmw32_kernel or mmp_kernel (dense matvec and matmul)",
     "attn": "attn_direct_kernel (FAST numerics, more than 4 lanes) / attn_partial_kernel (FAST split-context "
             "attention over the fp16 K/V cache)",
-    "head": "dmmv_kernel<T, NT, false> / from 5 lanes mmw_kernel<T, MT, false, ...> (output head)",
-    "qkv": "dmmv_self_kernel (1 lane) / dmmv_seg_kernel<NT> / from 5 lanes mmq_seg_kernel<1, SBW> "
+    "head": "dmmv_kernel<T, NT, false> / from 5 (Q4_K) or 8 (Q6_K) lanes mmw_kernel<T, MT, false, ...>, Q8_0 and Q4_0 "
+            "by size mmw32_kernel<T, false, ...> (output head)",
+    "qkv": "dmmv_self_kernel (1 lane) / dmmv_seg_kernel<NT> / K-quants from 5 lanes mmq_seg_kernel<1, SBW> "
            "(q, k, v in one launch)",
-    "wo": "dmmv_self_kernel or dmmv_kernel<T, NT, false> / from 5 to 8 lanes, by type, mmq_kernel<T, 1, false, SBW> "
-          "(wo + residual)",
+    "wo": "dmmv_self_kernel or dmmv_kernel<T, NT, false> / from 5 lanes or more, by type and size, "
+          "mmq_kernel<T, 1, false, SBW> or mmq32_kernel<T> (wo + residual)",
     "attn_scores": "attn_scores_kernel<HD> (PARITY, up to 4 lanes: dotF32-order scores with the q/k norm, rope and "
                    "K/V append) / attn_scores_many_kernel<HD> (more lanes: a thread per position, query elements "
                    "as scalar operands)",

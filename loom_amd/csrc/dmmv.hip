@@ -316,7 +316,9 @@ bool launch_dmmv_self(bool fused, DmmvSegParams sp, const float *x, int x_stride
     const int max_wgs = norm_w && cols <= SELF_MAX_COLS ? SELF_MAX_WGS_NORM : SELF_MAX_WGS;
     if (lds > 64 * 1024 || ((!norm_w || fused) && tiles > max_wgs)) // (the q/k/v launch: at any size)
         return false;
-    auto kern = fused ? dmmv_self_kernel<true, true> : norm_w ? dmmv_self_kernel<false, true> : dmmv_self_kernel<false, false>;
+    auto kern = fused    ? dmmv_self_kernel<true, true>
+                : norm_w ? dmmv_self_kernel<false, true>
+                         : dmmv_self_kernel<false, false>;
     hipLaunchKernelGGL(kern, dim3(tiles), dim3(256), lds, st, sp, x, x_stride, norm_w, eps, (int)part);
     note_launch();
     return true;

@@ -39,8 +39,9 @@ struct DmmvParams {
     int rpw;        // rows per wave
     int accumulate; // 1: out = out + value (a residual add, tensor.zig:50-52)
     int ident_n;    // launch_mmq only: > 0 means ident_n vectors in groups of consecutive
-                    // vectors, identity pair maps, plane 0 -- no group or pair table is read
-    // launch_mmq's streamed kernel (mmw_kernel) only:
+                    // vectors, plane 0: no group table and no pair_dst is read; pair_src must be
+                    // an identity table (the streamed and tiled kernels read it)
+    // launch_mmq's streamed kernels (mmw_kernel, mmw32_kernel) only:
     const int *group_src; // [n_groups][group_stride]: the vector of each group's t-th pair (past n: the
     int group_stride;     // last one's), read in place of pair_src at the group's index; null: pair_src
     int pos_ident;        // pair_dst (and, without group_src, pair_src) is the identity over pair positions

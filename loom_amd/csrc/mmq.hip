@@ -1726,8 +1726,10 @@ static bool lanes_streamed(int t, int rows, int cols, int n, bool fused) {
 // over nine streams per CU.  Measured, us per layer, one-shot / streamed gate/up
 // and down: 1024 x 512 x 32 top-4 Q4_K + Q6_K at 16 tokens (2304 streams each)
 // 32.3 / 34.4, at 19 33.9 / 35.6, at 24 (2432) 37.2 / 37.0, at 128 (4096) 49.7 /
-// 45.9; 2048 x 768 x 128 top-8 at 10 (8160 and 10880) 58.1 / 52.4.  The 32-value
-// blocks' one-shot form is slower at every size (63 / 41 at 24 tokens).
+// 45.9; 1024 x 1024 x 32 top-4 at 16 (4608 and 2304) 36.4 / 37.1; 1024 x 768 x 64 top-6
+// at 16 (6720 and 4480) 43.3 / 43.8, at 24 44.8 / 44.5; 1536 x 768 x 64 top-6 at 5
+// (2976 and 2976) 45.3 / 41.5; 2048 x 768 x 128 top-8 at 10 (8160 and 10880) 59.5 /
+// 51.5.  The 32-value blocks have no grouped one-shot form.
 constexpr long MMW_MIN_GROUP_STREAMS = 2400;
 static bool groups_few(int t, int rows, int n_groups, bool fused) {
     return is_k(t) && (long)n_groups * ((rows + 15) / 16) * (fused ? 2 : 1) < MMW_MIN_GROUP_STREAMS;
@@ -1804,9 +1806,10 @@ static bool lanes32_on_cores(int t, int rows, int cols, int n) {
 //     6.9, 8192 x 512 at 8 7.8 / 7.3;
 //   rows of 20 to 24 blocks, whose waves hold four blocks for three, from 2048
 //     rows: Q6_K 900 x 4864 at 9 13.4 / 12.7, 300 x 5120 12.5 / 13.3, 1900 x 6144
-//     14.5 / 15.1, 2500 x 6144 at 8 15.9 / 14.9; Q4_K only where the row's bytes are a multiple of
-//     the 128-byte line and under 8 vectors: 1000 x 6144 at 5 11.1 / 12.6, at 8
-//     14.6 / 13.2, 1000 x 5632 at 5 11.1 / 11.0.
+//     14.5 / 15.1, 2500 x 6144 at 8 15.9 / 14.9; Q4_K only where the row's bytes are a
+//     multiple of the 128-byte line and under 8 vectors: 1000 x 6144 at 5 11.1 / 12.6,
+//     at 8 14.6 / 13.2, 1000 x 5632 at 5 11.1 / 11.0.  Wider shapes (only streamed)
+//     from 512 pairs.
 static bool lanes_k_on_cores(int t, int rows, int cols, int n) {
     const int nb = cols / 256;
     if (n < (t == LH_Q4_K ? 5 : 8))
@@ -1820,13 +1823,12 @@ static bool lanes_k_on_cores(int t, int rows, int cols, int n) {
 
 // n vectors against one [rows][cols] matrix (or a fused pair): whether the
 // matrix cores take them from the dot4 matvec.  One matrix: lanes32_on_cores,
-// lanes_k_on_cores.  A shape only the streamed kernels serve needs 512 pairs.  A
-// fused pair, us per launch, dot4 / matrix cores: Q4_K from 16 (2048 x 7168 at 8 vectors
-// 16 / 24, at 24 47 / 25); Q8_0 / Q4_0, streamed only, us per call: 4096 x 2048
-// at 16 (256 pairs) 29.2 / 23.9 and 24.7 / 23.7, at 24 (512) 37.1 / 23.8 and
-// 33.4 / 23.7; 2048 x 2048 at 32 (256) 27.5 / 22.8 and 24.6 / 23.7, at 64 (512)
-// 44.2 / 23.0 and 42.2 / 23.9; 11008 x 4096 at 5 (688) 57.8 / 32.2 and 50.3 /
-// 32.8; 2048 x 7168 at 32 (256) 104 / 69 and 85 / 70.
+// lanes_k_on_cores.  A fused pair: Q4_K from 16 (us per launch, dot4 / matrix
+// cores: 2048 x 7168 at 8 vectors 16 / 24, at 24 47 / 25); Q8_0 / Q4_0, streamed
+// only, from 512 pairs (us per call: 4096 x 4096 at 8 (256) 31.5 / 31.8 and 27.6 /
+// 32.7; 4096 x 2048 at 16 (256) 29.2 / 23.9 and 24.7 / 23.7, at 24 (512) 37.1 / 23.8
+// and 33.4 / 23.7; 2048 x 2048 at 32 (256) 27.5 / 22.8 and 24.6 / 23.7, at 64 (512)
+// 44.2 / 23.0 and 42.2 / 23.9; 11008 x 4096 at 5 (688) 57.8 / 32.2 and 50.3 / 32.8).
 bool mmq_dense(int t, int rows, int cols, int n, bool fused) {
     if (rows < 1 || n < 1)
         return false;

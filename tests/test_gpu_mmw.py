@@ -1,10 +1,11 @@
 """GPU parity of the matrix-core matmuls that stream a row's blocks in order
 (mmw_kernel and, for 32-value blocks, mmw32_kernel, mmq.hip), of the one with 64
-x 128 tiles (mmp_kernel) and of the one-shot kernels beside them: bit-exact against per-vector oracle matvecs at the edges of its row tiles (16
-rows, 64 per work group), token sets (8) and groups (16, 32), block counts (odd
-and even, with the tokens' rows staged in LDS up to 2048 columns and not
-beyond), and at the extreme integers of its f16 mins and two-digit scales.
-Needs the GPU."""
+x 128 tiles (mmp_kernel) and of the one-shot kernels beside them: bit-exact
+against per-vector oracle matvecs at the edges of their row tiles (16 rows, 64
+per work group), token sets (8) and groups (16, 32), block counts (odd and even,
+with the tokens' rows staged in LDS up to 2048 columns and not beyond), at the
+extreme integers of the f16 mins and two-digit scales, and on either side of the
+lines between the kernels.  Needs the GPU."""
 import numpy as np
 import pytest
 
@@ -125,10 +126,11 @@ def test_streamed_32_block_matmul_edges(be, oracle, t, rows, cols, n):
 # either side of each line by which a Q8_0 / Q4_0 matmul is routed: rows on and off the 128-byte line (multiples
 # of 128 columns in Q8_0, 256 in Q4_0), widths of 1024, 1536 and 2048, one round of one-shot work groups and two
 @pytest.mark.parametrize("t", [Q4_0, Q8_0])
-@pytest.mark.parametrize("rows,cols,n", [(200, 4096, 16), (300, 3072, 7), (300, 3072, 8), (257, 1088, 8), (300, 1280, 9),
-                                         (768, 1024, 48), (768, 1024, 63), (1000, 960, 24), (2048, 512, 8),
+@pytest.mark.parametrize("rows,cols,n", [(200, 4096, 16), (300, 3072, 7), (300, 3072, 8), (257, 1088, 8),
+                                         (300, 1280, 9), (768, 1024, 48), (768, 1024, 63), (1000, 960, 24), (2048, 512, 8),
                                          (8192, 512, 12), (2500, 1536, 32), (2500, 1984, 32), (2500, 1984, 47),
-                                         (1500, 2016, 16), (6000, 2016, 12), (4096, 288, 8), (512, 160, 8), (512, 256, 9)])
+                                         (1500, 2016, 16), (6000, 2016, 12), (4096, 288, 8), (512, 160, 8),
+                                         (512, 256, 9)])
 def test_32_block_routes(be, oracle, t, rows, cols, n):
     rng = np.random.default_rng(rows + cols + n + t)
     raw = npref.pinned_scale_blocks(t, rows, cols, rng)
